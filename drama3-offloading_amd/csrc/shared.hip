@@ -14,20 +14,32 @@
 // moe_shared_gate_up computes a and s (one wave per intermediate row j,
 // holding the gate and up rows of j; one extra wave for the sigmoid gate
 // row), moe_shared_down the rest (4 output rows per wave) with the routed
-// output and the residual added in its epilogue.  Both are GEMVs over
-// weights read once per 4 tokens (per token at decode): HBM-bound, 6 MiB per
-// layer at H = 2048, Is = 512.  Sums are f32 fused multiply-adds over each
+// output and the residual added in its epilogue.  For one or two tokens both
+// are GEMVs over weights read once: HBM-bound, 6 MiB per layer at H = 2048,
+// Is = 512.  Sums are f32 fused multiply-adds over each
 // lane's 16-byte slices in row order, then the 64 lane sums (wave_sum_f32).
+//
+// From kSharedMmaFrom tokens both products run on the bf16 matrix cores
+// instead (the *_mma kernels below).
 #include "shared.hpp"
 
 namespace moe {
 
-constexpr int kSharedTB = 4;   // tokens per pass over the weights (1 when there is one)
+constexpr int kSharedTB = 2;   // tokens per pass over the weights (1 when there is one)
 constexpr int kUnroll = 4;     // 16-byte slices per lane in flight per row
 // Waves per workgroup: small workgroups spread the rows over every CU.  A
 // 1-token call (both kernels, 2048 x 512) measured 7.07 us at 2, 7.12 at 1
 // and 7.47 at 4 on MI355X.
 constexpr int kWavesPerWG = 2;
+
+// Fewest tokens of the matrix-core form.  Both kernels, H 2048, Is 512, a
+// graph over 40 layers' weights on MI355X, GEMV form -> matrix cores (us per
+// call, gate/up + down): 3 tokens 5.2 + 6.6 -> 4.8 + 3.8, 4 tokens 5.6 + 7.6
+// -> 5.0 + 3.8, 16 tokens 15.2 + 23.4 -> 5.9 + 3.9, 512 tokens 389 + 640 ->
+// 22.6 + 16.3.  One or two tokens stay on the GEMV form, whose sums the
+// decode launches that carry the shared expert reproduce.
+constexpr int kSharedMmaFrom = 3;
+constexpr int kSharedMmaMax = 16 * 65535;   // token tiles ride in the grid's y dimension
 
 template <int TB>
 __global__ __launch_bounds__(64 * kWavesPerWG) void shared_gate_up_kernel(
@@ -92,6 +104,182 @@ __global__ __launch_bounds__(64 * kWavesPerWG) void shared_down_kernel(
   }
 }
 
+// ------------------------------------------------------ on the matrix cores
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ v4f mfma_bf16_16x16x32(u32x4 a, u32x4 b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// One 64-wide K chunk of NR weight rows' tiles against TT token tiles: lane
+// (q, i) holds K 16q .. 16q + 15 of row i of each tile, two MFMAs a product.
+template <int NR, int TT>
+struct MmaChunk {
+  u32x4 a[NR][2], b[TT][2];
+  __device__ __forceinline__ void load(const uint16_t* const (&rows)[NR],
+                                       const uint16_t* const (&toks)[TT], int64_t o) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      b[t][0] = load16(toks[t] + o);
+      b[t][1] = load16(toks[t] + o + 8);
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      a[r][0] = load16(rows[r] + o);
+      a[r][1] = load16(rows[r] + o + 8);
+    }
+  }
+  // live false: a chunk past the end (its loads re-read the last one) adds nothing
+  __device__ __forceinline__ void fold(v4f (&acc)[NR][TT], bool live) {
+    const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const u32x4 av = live ? a[r][h] : z;
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+          acc[r][t] = mfma_bf16_16x16x32(av, live ? b[t][h] : z, acc[r][t]);
+      }
+    }
+  }
+};
+
+// Gate and up rows of NR * 8 intermediate columns against 16 * TT tokens: one
+// 16-row tile (NR 1) is 8 gate rows and the 8 up rows of the same columns,
+// two (NR 2) are 16 of each.  The workgroup's W waves split K (wave v takes
+// the 64-wide chunks v, v + W, ...), U chunks in flight each, and their
+// partial tiles are added in wave order through LDS.  The last workgroup
+// column (blockIdx.x * NR * 8 == inter) is the sigmoid gate row: all rows of
+// its tiles are that row.
+template <int NR, int TT, int W, int U>
+__global__ __launch_bounds__(64 * W) void shared_gate_up_mma_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ wg, const uint16_t* __restrict__ wu,
+    const uint16_t* __restrict__ wsg, int32_t tokens, int32_t hidden, int32_t inter,
+    uint16_t* __restrict__ act, float* __restrict__ sig) {
+  constexpr int NJ = NR * 8;                      // columns per workgroup
+  __shared__ float part[W][NR][TT][16][17];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int i = lane & 15, q = lane >> 4;
+  const int j0 = static_cast<int>(blockIdx.x) * NJ;
+  const int t0 = static_cast<int>(blockIdx.y) * 16 * TT;
+  const bool gate_row = j0 >= inter;
+  const uint16_t* rows[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const bool up = NR == 1 ? i >= 8 : r == 1;
+    const int j = j0 + (NR == 1 ? i & 7 : i);
+    rows[r] = (gate_row ? wsg : (up ? wu : wg) + static_cast<int64_t>(j) * hidden) + 16 * q;
+  }
+  const uint16_t* toks[TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+    toks[t] = x + static_cast<int64_t>(min(t0 + 16 * t + i, tokens - 1)) * hidden + 16 * q;
+  const int nchunk = hidden >> 6;                 // hidden % 128 == 0
+  v4f acc[NR][TT];
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc[r][t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int c0 = wave; c0 < nchunk; c0 += W * U) {
+    MmaChunk<NR, TT> ch[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      ch[u].load(rows, toks, static_cast<int64_t>(min(c0 + u * W, nchunk - 1)) * 64);
+    __builtin_amdgcn_sched_barrier(0);            // every load is issued before the math below
+#pragma unroll
+    for (int u = 0; u < U; ++u) ch[u].fold(acc, c0 + u * W < nchunk);
+  }
+  // lane (q, i) holds rows 4q .. 4q + 3 of token column i
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) part[wave][r][t][4 * q + k][i] = acc[r][t][k];
+  __syncthreads();
+  for (int o = threadIdx.x; o < TT * 16 * NJ; o += 64 * W) {
+    const int rr = o % NJ, tc = (o / NJ) & 15, t = o / (16 * NJ);
+    const int ur = NR == 1 ? rr + 8 : rr;         // the up row of column rr in its tile
+    float g = part[0][0][t][rr][tc], u = part[0][NR - 1][t][ur][tc];
+#pragma unroll
+    for (int v = 1; v < W; ++v) {
+      g += part[v][0][t][rr][tc];
+      u += part[v][NR - 1][t][ur][tc];
+    }
+    const int tok = t0 + 16 * t + tc;
+    if (tok >= tokens) continue;
+    if (!gate_row)
+      act[static_cast<int64_t>(tok) * inter + j0 + rr] = shared_act(g, u);
+    else if (rr == 0)
+      sig[tok] = shared_sig(g);
+  }
+}
+
+// Down: a wave takes 16 output rows against 16 * TT tokens over all of K, so
+// nothing is exchanged between waves; W waves of consecutive rows share the
+// tokens' activations through the cache.  Lane (q, i) ends with outputs
+// 4q .. 4q + 3 of token i, moved as one 8-byte unit where the buffers allow
+// it (vec: routed, residual and out 8-byte aligned).
+template <int TT, int W, int U>
+__global__ __launch_bounds__(64 * W) void shared_down_mma_kernel(
+    const uint16_t* __restrict__ act, const float* __restrict__ sig,
+    const uint16_t* __restrict__ wd, int32_t tokens, int32_t hidden, int32_t inter, int vec,
+    const uint16_t* routed, const uint16_t* residual, uint16_t* out) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int i = lane & 15, q = lane >> 4;
+  const int r0 = (static_cast<int>(blockIdx.x) * W + wave) * 16;
+  if (r0 >= hidden) return;                       // the whole wave; no barrier below
+  const int t0 = static_cast<int>(blockIdx.y) * 16 * TT;
+  const uint16_t* const rows[1] = {wd + static_cast<int64_t>(r0 + i) * inter + 16 * q};
+  const uint16_t* toks[TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+    toks[t] = act + static_cast<int64_t>(min(t0 + 16 * t + i, tokens - 1)) * inter + 16 * q;
+  const int nchunk = inter >> 6;                  // inter % 128 == 0
+  v4f acc[1][TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t) acc[0][t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int c0 = 0; c0 < nchunk; c0 += U) {
+    MmaChunk<1, TT> ch[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      ch[u].load(rows, toks, static_cast<int64_t>(min(c0 + u, nchunk - 1)) * 64);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) ch[u].fold(acc, c0 + u < nchunk);
+  }
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const int tok = t0 + 16 * t + i;
+    if (tok >= tokens) continue;
+    const int64_t o = static_cast<int64_t>(tok) * hidden + r0 + 4 * q;
+    const float sg = sig[tok];
+    uint16_t rv[4] = {0, 0, 0, 0}, sv[4] = {0, 0, 0, 0}, ov[4];
+    if (vec) {
+      if (routed) __builtin_memcpy(rv, __builtin_assume_aligned(routed + o, 8), 8);
+      if (residual) __builtin_memcpy(sv, __builtin_assume_aligned(residual + o, 8), 8);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (routed) rv[k] = routed[o + k];
+        if (residual) sv[k] = residual[o + k];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      ov[k] = shared_out(acc[0][t][k], sg, routed != nullptr, rv[k], residual != nullptr, sv[k]);
+    if (vec) {
+      __builtin_memcpy(__builtin_assume_aligned(out + o, 8), ov, 8);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) out[o + k] = ov[k];
+    }
+  }
+}
+
 // flag = 1 when every element of x is finite, else 0.  One workgroup, so the
 // flag is written exactly once and needs no clearing before (a graph replays
 // it as is).
@@ -123,9 +311,44 @@ __global__ __launch_bounds__(1024) void all_finite_kernel(const void* __restrict
   if (threadIdx.x == 0) *flag = all ? 1 : 0;
 }
 
+template <int NR, int TT, int W, int U>
+static void launch_gate_up_mma(const uint16_t* x, const uint16_t* wg, const uint16_t* wu,
+                               const uint16_t* wsg, int32_t tokens, int32_t hidden, int32_t inter,
+                               uint16_t* act, float* sig, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(inter / (NR * 8) + 1),
+                  static_cast<unsigned>((tokens + 16 * TT - 1) / (16 * TT)));
+  hipLaunchKernelGGL((shared_gate_up_mma_kernel<NR, TT, W, U>), grid, dim3(64 * W), 0, s, x, wg,
+                     wu, wsg, tokens, hidden, inter, act, sig);
+}
+
+template <int TT, int W, int U>
+static void launch_down_mma(const uint16_t* act, const float* sig, const uint16_t* wd,
+                            int32_t tokens, int32_t hidden, int32_t inter, int vec,
+                            const uint16_t* routed, const uint16_t* residual, uint16_t* out,
+                            hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>((hidden + 16 * W - 1) / (16 * W)),
+                  static_cast<unsigned>((tokens + 16 * TT - 1) / (16 * TT)));
+  hipLaunchKernelGGL((shared_down_mma_kernel<TT, W, U>), grid, dim3(64 * W), 0, s, act, sig, wd,
+                     tokens, hidden, inter, vec, routed, residual, out);
+}
+
 int launch_shared_gate_up(const uint16_t* x, const uint16_t* wg, const uint16_t* wu,
                           const uint16_t* wsg, int32_t tokens, int32_t hidden, int32_t inter,
                           uint16_t* act, float* sig, hipStream_t s) {
+  if (tokens >= kSharedMmaFrom && tokens <= kSharedMmaMax) {
+    // Small calls are one round trip to memory, spread over as many CUs as
+    // there are tiles (8 columns, 16 tokens); larger ones re-read the weights
+    // and x from the L2, so the tiles grow.  us at 32 / 64 / 128 / 512 tokens
+    // for <1,1,8,4>: 6.0 / 9.3 / 13.0 / 34.8; <1,2,8,2>: 7.9 / 8.0 / 13.0 /
+    // 30.3; <2,2,8,2>: 9.7 / 9.7 / 9.9 / 22.6.
+    if (tokens <= 32)
+      launch_gate_up_mma<1, 1, 8, 4>(x, wg, wu, wsg, tokens, hidden, inter, act, sig, s);
+    else if (tokens <= 64)
+      launch_gate_up_mma<1, 2, 8, 2>(x, wg, wu, wsg, tokens, hidden, inter, act, sig, s);
+    else
+      launch_gate_up_mma<2, 2, 8, 2>(x, wg, wu, wsg, tokens, hidden, inter, act, sig, s);
+    return check_launch("moe_shared_gate_up");
+  }
   const unsigned grid = static_cast<unsigned>((inter + 1 + kWavesPerWG - 1) / kWavesPerWG);
   auto kern = tokens == 1 ? shared_gate_up_kernel<1> : shared_gate_up_kernel<kSharedTB>;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kWavesPerWG), 0, s, x, wg, wu, wsg, tokens,
@@ -136,6 +359,17 @@ int launch_shared_gate_up(const uint16_t* x, const uint16_t* wg, const uint16_t*
 int launch_shared_down(const uint16_t* act, const float* sig, const uint16_t* wd, int32_t tokens,
                        int32_t hidden, int32_t inter, const uint16_t* routed,
                        const uint16_t* residual, uint16_t* out, hipStream_t s) {
+  if (tokens >= kSharedMmaFrom && tokens <= kSharedMmaMax) {
+    auto al8 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; };
+    const int vec = al8(routed) && al8(residual) && al8(out);
+    // us at 16 / 128 / 256 / 512 / 1024 tokens: <1,1,8> 3.9 / 6.6 / 11.2 /
+    // 19.0 / 34.2, <2,4,4> 6.9 / 9.3 / 10.2 / 16.3 / 27.8
+    if (tokens <= 128)
+      launch_down_mma<1, 1, 8>(act, sig, wd, tokens, hidden, inter, vec, routed, residual, out, s);
+    else
+      launch_down_mma<2, 4, 4>(act, sig, wd, tokens, hidden, inter, vec, routed, residual, out, s);
+    return check_launch("moe_shared_down");
+  }
   // one 16-byte slice per lane and row covers inter <= 512: no batch to fill
   const bool one = inter <= 512;
   auto kern = tokens == 1 ? (one ? shared_down_kernel<1, 1> : shared_down_kernel<1, kUnroll>)

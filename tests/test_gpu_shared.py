@@ -64,6 +64,53 @@ def test_shared_expert_matches_oracle(lib, dev, T, H, Is):
     assert same >= 0.99 and ulps <= 2.0
 
 
+@pytest.mark.parametrize("T,H,Is", [(4, 384, 640), (16, 2048, 512), (17, 128, 128), (32, 640, 384),
+                                    (33, 2048, 512), (64, 384, 128), (65, 640, 256),
+                                    (128, 128, 640), (129, 2048, 512), (300, 1152, 384)])
+def test_shared_matrix_core_shapes(lib, dev, T, H, Is):
+    """The matrix-core form at the edges of its token tiles and at widths
+    that leave its K split and its row tiles uneven, with the down half's
+    buffers 8-byte aligned and not (an element's offset): the bar of
+    test_shared_expert_matches_oracle, and nothing written past the tokens.
+
+    act = silu(g) * u of sums that cancel has no bound in ulps of itself: a
+    product of bf16 values is exact in float32 and a wave's chain is at most
+    H / 8 + 8 float32 additions, so each sum may be off by (H / 8 + 8) *
+    2^-24 of the sum of its products' magnitudes before it is rounded, and
+    act by that through silu (slope at most 1.1) and the product; the ulps
+    are counted beyond it.  The sigmoid and the down half are judged as they
+    stand (sigmoid's argument enters absolutely, the residual is of order 1)."""
+    p = _weights(T + H + Is, T, H, Is, dev)
+    act = torch.full((T + 1, Is), 7.0, dtype=torch.bfloat16, device=dev)
+    sig = torch.full((T + 1,), 7.0, dtype=torch.float32, device=dev)
+    say(f"shared expert, matrix cores: T={T} H={H} Is={Is}")
+    lib.shared_gate_up(p["x"], p["wg"], p["wu"], p["wsg"], act[:T], sig[:T])
+    outs = []
+    for off in (0, 1):
+        flat = torch.full((T * H + off + 1,), 7.0, dtype=torch.bfloat16, device=dev)
+        lib.shared_down(act[:T], sig[:T], p["wd"], flat[off:off + T * H].view(T, H),
+                        routed=p["routed"], residual=p["res"])
+        torch.cuda.synchronize()
+        assert bool((flat[:off] == 7).all()) and float(flat[-1]) == 7
+        outs.append(flat[off:off + T * H].view(T, H).clone())
+    assert bool((act[T] == 7).all()) and float(sig[T]) == 7
+    assert torch.equal(outs[0], outs[1])
+    q = {k: _np(v) for k, v in p.items()}
+    want_a, want_s = shared.gate_up(q["x"], q["wg"], q["wu"], q["wsg"])
+    got_a, got_s = _np(act[:T]), sig[:T].cpu().numpy()
+    d = [(H / 8 + 8) * 2.0 ** -24 * (np.abs(q["x"]) @ np.abs(q[w]).T) for w in ("wg", "wu")]
+    g, u = (q["x"].astype(np.float64) @ q[w].T.astype(np.float64) for w in ("wg", "wu"))
+    slack = 1.1 * d[0] * (np.abs(u) + d[1]) + np.abs(g) * d[1]
+    off = got_a.astype(np.float64) - want_a
+    near = want_a + np.sign(off) * np.maximum(np.abs(off) - slack, 0.0)
+    assert float((got_a == want_a).mean()) >= 0.99
+    for name, got, want in (("act", near, want_a), ("sig", got_s, want_s),
+                            ("down", _np(outs[0]), shared.down(got_a, got_s, q["wd"], q["routed"],
+                                                               q["res"]))):
+        same, ulps = _agree(got, want)
+        assert same >= 0.99 and ulps <= 2.0, (name, same, ulps)
+
+
 def test_shared_down_in_place(lib, dev):
     """out may alias routed (the decode step writes the block sum over it)."""
     T, H, Is = 2, 512, 256
