@@ -403,8 +403,8 @@ __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
     if (blockIdx.y == 0) commit_table(cm);
     return;
   }
-  __shared__ __align__(16) uint8_t aq[kMaxK][kMaxInter];
-  __shared__ float as_[kMaxK][kMaxInter / 128];
+  // aq [2 * kwaves][inter] e4m3, then as_ [2 * kwaves][inter / 128] f32
+  extern __shared__ __align__(16) uint8_t down_smem[];
   __shared__ __align__(16) float part[kMaxK + 1][kDownRows];   // [kMaxK]: discarded quadrants
   __shared__ float wpart[kMaxK];
   __shared__ float spart[SHARED ? kDownRows : 1];
@@ -415,6 +415,8 @@ __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
   const int t = blockIdx.y;
   const int c0 = blockIdx.x * kDownRows;
   const int kwaves = (top_k + 1) >> 1;
+  uint8_t* const aq = down_smem;
+  float* const as_ = reinterpret_cast<float*>(down_smem + 2 * kwaves * inter);
   if (SHARED && wave == kwaves) {
     // the shared expert's 8 down rows of this workgroup, token t
     const uint16_t* rows[kDownRows];
@@ -494,20 +496,24 @@ __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
     a[c] = load_op_nt(wrow + (c < Gi ? c : Gi - 1) * ow.kstep, ow.half);
   __builtin_amdgcn_sched_barrier(0);   // every load above is issued before the math below
   // both pairs' activations, quantised per 128 into LDS: 16 lanes x 8
-  quantize8_f32(araw0, lane * 8 < inter, lane * 8, aq[k0], as_[k0]);
-  quantize8_f32(araw1, lane * 8 < inter, lane * 8, aq[k0 + 1], as_[k0 + 1]);
+  uint8_t* const aq0 = aq + k0 * inter;
+  uint8_t* const aq1 = aq0 + inter;
+  float* const as0 = as_ + k0 * (inter >> 7);
+  float* const as1 = as0 + (inter >> 7);
+  quantize8_f32(araw0, lane * 8 < inter, lane * 8, aq0, as0);
+  quantize8_f32(araw1, lane * 8 < inter, lane * 8, aq1, as1);
   for (int base = 512; base < inter; base += 512) {
     const int j = base + lane * 8;
     const int jj = j < inter ? j : 0;
     float4 ar[2];
     ar[0] = *reinterpret_cast<const float4*>(ap0 + jj);
     ar[1] = *reinterpret_cast<const float4*>(ap0 + jj + 4);
-    quantize8_f32(ar, j < inter, j, aq[k0], as_[k0]);
+    quantize8_f32(ar, j < inter, j, aq0, as0);
     ar[0] = *reinterpret_cast<const float4*>(ap1 + jj);
     ar[1] = *reinterpret_cast<const float4*>(ap1 + jj + 4);
-    quantize8_f32(ar, j < inter, j, aq[k0 + 1], as_[k0 + 1]);
+    quantize8_f32(ar, j < inter, j, aq1, as1);
   }
-  // aq[k0..k0+1] and as_[k0..k0+1] are this wave's own: its LDS accesses
+  // the aq and as_ rows k0, k0 + 1 are this wave's own: its LDS accesses
   // complete in order, so a wave-scope fence (which keeps the compiler from
   // moving the reads above the writes) replaces a workgroup barrier
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -516,8 +522,8 @@ __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
 
   // B operand: this lane's column is its slot's activation; the row sums
   // of slot dhalf run in K-block order with that slot's scales
-  const uint8_t* bq = aq[k0 + half];
-  const float* asd = as_[k0 + dhalf];
+  const uint8_t* bq = half ? aq1 : aq0;
+  const float* asd = dhalf ? as1 : as0;
   v4f acc = {0.f, 0.f, 0.f, 0.f};
   for (int g0 = 0; g0 < Gi; g0 += kDownChunk) {
     if (g0 > 0) {
@@ -638,9 +644,9 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_a16_kernel(
     const uint8_t* __restrict__ w13, const float* __restrict__ s13, int64_t w13_es,
     int64_t s13_es, int tiled, int32_t n_experts, int32_t hidden, int32_t inter,
     float* __restrict__ act) {
-  __shared__ __align__(16) uint16_t xb[kMaxHidden];
-  __shared__ __align__(16) float dpart[kGateUpTiles][kMaxHidden / 128][16];
-  __shared__ float spart[kGateUpTiles][kMaxHidden / 128];
+  // x[t] [hidden] bf16, then per tile the block products [G][16] f32, then
+  // their scales [G] f32
+  extern __shared__ __align__(16) uint16_t xb[];
   __shared__ __align__(16) float upsum[16];
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
@@ -661,6 +667,8 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_a16_kernel(
   const int tile = wu / kGateUpSplit;
   const int part = wu % kGateUpSplit;
   const bool owner = part == 0;
+  float* const dpart = reinterpret_cast<float*>(xb + hidden) + tile * G * 16;
+  float* const spart = reinterpret_cast<float*>(xb + hidden) + (kGateUpTiles * 16 + tile) * G;
   const int Gs = (G + kGateUpSplit - 1) / kGateUpSplit;
   const int gb = min(part * Gs, G);
   const int gn = min(gb + Gs, G) - gb;
@@ -712,8 +720,8 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_a16_kernel(
           block_fma(acc, d, sw[c]);
         } else {
           // every lane stores (see gateup_gemv_kernel)
-          *reinterpret_cast<float4*>(&dpart[tile][g][4 * q]) = make_float4(d[0], d[1], d[2], d[3]);
-          spart[tile][g] = sw[c];
+          *reinterpret_cast<float4*>(dpart + g * 16 + 4 * q) = make_float4(d[0], d[1], d[2], d[3]);
+          spart[g] = sw[c];
         }
       }
     }
@@ -722,9 +730,9 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_a16_kernel(
   if (owner) {
 #pragma unroll 8
     for (int g = gn; g < G; ++g) {
-      const float4 d = *reinterpret_cast<const float4*>(&dpart[tile][g][4 * q]);
+      const float4 d = *reinterpret_cast<const float4*>(dpart + g * 16 + 4 * q);
       const v4f dv = {d.x, d.y, d.z, d.w};
-      block_fma(acc, dv, spart[tile][g]);
+      block_fma(acc, dv, spart[g]);
     }
     if (tile == 1)
       *reinterpret_cast<float4*>(&upsum[4 * q]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
@@ -747,7 +755,7 @@ __global__ __launch_bounds__(64 * (kMaxK / 2)) void down_gemv_a16_kernel(
     const float* __restrict__ s2, int64_t w2_es, int64_t s2_es, int tiled, int32_t n_experts,
     int32_t hidden, int32_t inter, const uint16_t* __restrict__ residual,
     uint16_t* __restrict__ out) {
-  __shared__ __align__(16) uint16_t ab[kMaxK][kMaxInter];
+  extern __shared__ __align__(16) uint16_t ab[];    // [2 * kwaves][inter] bf16
   __shared__ __align__(16) float part[kMaxK + 1][kDownRows];
   __shared__ float wpart[kMaxK];
   const int wave = threadIdx.x >> 6;
@@ -810,23 +818,25 @@ __global__ __launch_bounds__(64 * (kMaxK / 2)) void down_gemv_a16_kernel(
       *reinterpret_cast<uint4*>(dst + j) = v;
     }
   };
-  put8(araw0, lane * 8, ab[k0]);
-  put8(araw1, lane * 8, ab[k0 + 1]);
+  uint16_t* const ab0 = ab + k0 * inter;
+  uint16_t* const ab1 = ab0 + inter;
+  put8(araw0, lane * 8, ab0);
+  put8(araw1, lane * 8, ab1);
   for (int base = 512; base < inter; base += 512) {
     const int j = base + lane * 8;
     const int jj = j < inter ? j : 0;
     float4 ar[2];
     ar[0] = *reinterpret_cast<const float4*>(ap0 + jj);
     ar[1] = *reinterpret_cast<const float4*>(ap0 + jj + 4);
-    put8(ar, j, ab[k0]);
+    put8(ar, j, ab0);
     ar[0] = *reinterpret_cast<const float4*>(ap1 + jj);
     ar[1] = *reinterpret_cast<const float4*>(ap1 + jj + 4);
-    put8(ar, j, ab[k0 + 1]);
+    put8(ar, j, ab1);
   }
   // the wave's own rows: a wave-scope fence stands for a barrier (see down_gemv_kernel)
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  const uint16_t* bq = ab[k0 + half];
+  const uint16_t* bq = half ? ab1 : ab0;
   v4f acc = {0.f, 0.f, 0.f, 0.f};
   for (int g0 = 0; g0 < Gi; g0 += kDownChunk) {
     if (g0 > 0) {
@@ -871,6 +881,23 @@ __global__ __launch_bounds__(64 * (kMaxK / 2)) void down_gemv_a16_kernel(
     if (residual) y = f32_to_bf16(bf16_to_f32(res_v) + bf16_to_f32(y));
     out[o] = y;
   }
+}
+
+// LDS of one workgroup of the down launches and of the bf16-activation
+// gate/up launch, sized by the call instead of by the largest call served:
+// with room for 16 experts of inter 2048 a workgroup held 34 KiB (66 KiB with
+// bf16 activations), which let 4 (2) of them onto a CU that has wave slots for
+// 8, and left batches of several tokens short of loads in flight: a
+// bf16-activation call of 12 tokens (H 2048, I 512, top-8 of 256) took 56.3 us
+// with the fixed arrays and takes 51.1; an e4m3 one of 8 tokens gains 1 %.
+static unsigned down_lds(int32_t top_k, int32_t inter) {
+  return static_cast<unsigned>(2 * ((top_k + 1) / 2) * (inter + (inter >> 7) * 4));
+}
+static unsigned down_a16_lds(int32_t top_k, int32_t inter) {
+  return static_cast<unsigned>(2 * ((top_k + 1) / 2) * inter * 2);
+}
+static unsigned gateup_a16_lds(int32_t hidden) {
+  return static_cast<unsigned>(hidden * 2 + kGateUpTiles * (hidden >> 7) * 17 * 4);
 }
 
 // The two decode launches; `sh` (nullable) carries the shared expert along.
@@ -930,12 +957,12 @@ static int launch_gemv(const uint16_t* x, const void* ids, int ids64, const void
   if (sh) {
     hipLaunchKernelGGL(down_gemv_kernel<true>, dim3(hidden / kDownRows, tokens),
                        dim3(64 * ((top_k + 1) / 2 + 1)),
-                       0, s, h, ids, ids64, weights, wbf16, top_k, w2, s2, es.w2, es.s2,
-                       static_cast<int>(es.layout), n_experts, hidden, inter, residual, out, *sh,
+                       down_lds(top_k, inter), s, h, ids, ids64, weights, wbf16, top_k, w2, s2,
+                       es.w2, es.s2, static_cast<int>(es.layout), n_experts, hidden, inter, residual, out, *sh,
                        TableCommit{});
   } else {
     hipLaunchKernelGGL(down_gemv_kernel<false>, dim3(hidden / kDownRows, tokens),
-                       dim3(64 * ((top_k + 1) / 2)), 0, s,
+                       dim3(64 * ((top_k + 1) / 2)), down_lds(top_k, inter), s,
                        h, ids, ids64, weights, wbf16, top_k, w2, s2, es.w2, es.s2,
                        static_cast<int>(es.layout), n_experts, hidden, inter, residual, out,
                        SharedRefs{}, TableCommit{});
@@ -953,14 +980,14 @@ static int launch_gemv_a16(const uint16_t* x, const void* ids, int ids64, const 
   const int64_t pairs = static_cast<int64_t>(tokens) * top_k;
   const unsigned gx = static_cast<unsigned>((2 * inter) / 16);
   hipLaunchKernelGGL(gateup_gemv_a16_kernel, dim3(gx / kGateUpTiles, pairs),
-                     dim3(64 * kGateUpWaves), 0, s, x, ids, ids64, top_k, w13, s13, es.w13,
-                     es.s13, static_cast<int>(es.layout), n_experts, hidden, inter, h);
+                     dim3(64 * kGateUpWaves), gateup_a16_lds(hidden), s, x, ids, ids64, top_k, w13,
+                     s13, es.w13, es.s13, static_cast<int>(es.layout), n_experts, hidden, inter, h);
   int rc = check_launch("moe_fp8_moe_forward(gate/up, bf16 activations)");
   if (rc) return rc;
   hipLaunchKernelGGL(down_gemv_a16_kernel, dim3(hidden / kDownRows, tokens),
-                     dim3(64 * ((top_k + 1) / 2)), 0, s, h, ids, ids64, weights, wbf16, top_k, w2,
-                     s2, es.w2, es.s2, static_cast<int>(es.layout), n_experts, hidden, inter,
-                     residual, out);
+                     dim3(64 * ((top_k + 1) / 2)), down_a16_lds(top_k, inter), s, h, ids, ids64,
+                     weights, wbf16, top_k, w2, s2, es.w2, es.s2, static_cast<int>(es.layout),
+                     n_experts, hidden, inter, residual, out);
   return check_launch("moe_fp8_moe_forward(down, bf16 activations)");
 }
 
@@ -973,13 +1000,13 @@ int launch_down_gemv(const float* act, const int32_t* slots, const void* weights
   const unsigned extra = commit ? 1u : 0u;
   if (sh) {
     hipLaunchKernelGGL(down_gemv_kernel<true>, dim3(hidden / kDownRows + extra, tokens),
-                       dim3(64 * ((top_k + 1) / 2 + 1)), 0, s, act, slots, 0, weights, wbf16,
-                       top_k, w2, s2, w2_es, s2_es, tiled, n_slots, hidden, inter, residual, out,
+                       dim3(64 * ((top_k + 1) / 2 + 1)), down_lds(top_k, inter), s, act, slots, 0,
+                       weights, wbf16, top_k, w2, s2, w2_es, s2_es, tiled, n_slots, hidden, inter, residual, out,
                        *sh, cm);
   } else {
     hipLaunchKernelGGL(down_gemv_kernel<false>, dim3(hidden / kDownRows + extra, tokens),
-                       dim3(64 * ((top_k + 1) / 2)), 0, s, act, slots, 0, weights, wbf16, top_k,
-                       w2, s2, w2_es, s2_es, tiled, n_slots, hidden, inter, residual, out,
+                       dim3(64 * ((top_k + 1) / 2)), down_lds(top_k, inter), s, act, slots, 0, weights,
+                       wbf16, top_k, w2, s2, w2_es, s2_es, tiled, n_slots, hidden, inter, residual, out,
                        SharedRefs{}, cm);
   }
   return check_launch("down_gemv_kernel");

@@ -67,6 +67,8 @@ def _forward(lib, dev, host, x, ids, w, mode, ids_dtype=torch.int64, w_dtype=tor
     (2, 4, 8192, 2048, 1, 4),      # the kernels' limits
     (3, 6, 640, 384, 4, 3),        # K-blocks not a multiple of the chunk, odd top_k
     (4, 16, 2048, 512, 20, 5),     # more tokens than mode 0 would send to the GEMV
+    (5, 16, 128, 2048, 3, 16),     # the down launches' LDS at its largest, and an odd slot of it
+    (6, 16, 256, 1920, 2, 15),
 ], ids=lambda c: f"E{c[1]}-H{c[2]}-I{c[3]}-T{c[4]}-K{c[5]}")
 def test_a16_matches_the_dequantise_path(lib, dev, case):
     seed, E, H, I, T, K = case
