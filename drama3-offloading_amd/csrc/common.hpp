@@ -286,6 +286,20 @@ __device__ __forceinline__ v8i load_op_nt(const uint8_t* p, int half) {
   return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
 }
 
+// The same operand through the caches, where several workgroups read it.
+__device__ __forceinline__ v8i load_op(const uint8_t* p, int half) {
+  const u32x4 lo = *reinterpret_cast<const u32x4*>(p);
+  const u32x4 hi = *reinterpret_cast<const u32x4*>(p + half);
+  return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+}
+
+// 32-byte MFMA operand from two 16-byte units of LDS.
+__device__ __forceinline__ v8i lds_op32(const uint8_t* p0, const uint8_t* p1) {
+  const u32x4 lo = *reinterpret_cast<const u32x4*>(p0);
+  const u32x4 hi = *reinterpret_cast<const u32x4*>(p1);
+  return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+}
+
 // acc += d * sc with one fused multiply-add (one rounding) per element,
 // written out so that every kernel rounds its block sums identically.
 __device__ __forceinline__ void block_fma(v4f& acc, const v4f& d, float sc) {

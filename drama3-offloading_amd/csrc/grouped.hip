@@ -104,13 +104,6 @@ struct StreamArgs {
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-// 32-byte MFMA operand from two 16-byte units of LDS.
-__device__ __forceinline__ v8i lds_op32(const uint8_t* p0, const uint8_t* p1) {
-  const u32x4 lo = *reinterpret_cast<const u32x4*>(p0);
-  const u32x4 hi = *reinterpret_cast<const u32x4*>(p1);
-  return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-}
-
 // The GLU form of the gate/up projection.  An item takes intermediate
 // columns [c, c + 32*GPW) -- whole 128-column groups, GPW >= 4 -- with their
 // gate rows (waves 0-1) and their up rows (waves 2-3), so it holds every
@@ -355,16 +348,16 @@ constexpr int kDownShape = 3;         // (8, 8)
 static_assert(kGateUpShape < kNumShapes && kDownShape < kNumShapes, "shape index");
 
 // Expected tile count of P uniform picks over n_experts: each expert's
-// pair count n is Poisson(P / n_experts) and takes ceil(n / 32) tiles,
-// E[ceil(n / 32)] = sum over j >= 0 of P(n > 32 j).
-static double expected_tiles(int64_t P, int32_t n_experts) {
+// pair count n is Poisson(P / n_experts) and takes ceil(n / rows) tiles,
+// E[ceil(n / rows)] = sum over j >= 0 of P(n > rows * j).
+static double expected_tiles(int64_t P, int32_t n_experts, int rows) {
   if (P <= 0) return 0.0;
   const double lam = static_cast<double>(P) / n_experts;
-  if (lam > 1000.0) return n_experts * (lam / kTileTok + 0.5);
+  if (lam > 1000.0) return n_experts * (lam / rows + 0.5);
   double tiles = 0.0, cdf = 0.0, logp = -lam;   // log P(n = 0)
   int n = 0;
   for (int j = 0;; ++j) {
-    const int m = kTileTok * j;
+    const int m = rows * j;
     for (; n <= m; ++n) {
       cdf += exp(logp);
       logp += log(lam) - log(static_cast<double>(n + 1));
@@ -385,7 +378,7 @@ static double expected_tiles(int64_t P, int32_t n_experts) {
 // I 512, T = 17 .. 1024 tokens and every pair of shapes: gate/up (16, 4)
 // with down (8, 8) was the fastest pair or within 1.5 % of it at every T.
 static int pick_shape(int64_t P, int32_t n_experts, int32_t rows, int target) {
-  const double tiles = expected_tiles(P, n_experts);
+  const double tiles = expected_tiles(P, n_experts, kTileTok);
   int fallback = -1;
   for (int i = target; i >= 0; --i) {
     const int g = kShapes[i].gpw;
@@ -450,6 +443,64 @@ __global__ __launch_bounds__(512) void grouped_silu_kernel(const float* __restri
 }
 
 
+// Calls on the wide tiles (grouped_wide.hip): from 18 rows per expert, with w2
+// in whole row blocks.  us per call at H 2048, I 512, tile order, streamed ->
+// wide, MI355X: 256 experts top-8, 512 tokens (16 rows per expert) 159.7 ->
+// 162.0, 700 182 -> 171, 1021 216 -> 181, 2000 328 -> 258, 4096 574 -> 393;
+// 64 experts top-6, 200 tokens (19) 61.3 -> 54.5, 700 101 -> 75; 16 experts
+// top-8, 100 tokens 44.4 -> 40.6; row order, 1021 tokens 276 -> 208.
+constexpr int kWideRowsPerExpert = 18;
+static bool use_wide(int64_t P, int32_t n_experts, int32_t hidden) {
+  return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(kWideRowsPerExpert) * n_experts;
+}
+
+static int launch_wide(const GroupedLayout& L, char* ws, int64_t P, int32_t top_k,
+                       const uint8_t* w13, const float* s13, const uint8_t* w2, const float* s2,
+                       const moe_expert_strides& es, int32_t n_experts, int32_t hidden,
+                       int32_t inter, hipStream_t s) {
+  const int64_t max_tiles = (P + kWideTile - 1) / kWideTile + n_experts;
+  const double tiles = expected_tiles(P, n_experts, kWideTile);
+  WideArgs A{};
+  A.act = reinterpret_cast<const uint8_t*>(ws + L.xq);
+  A.act_s = reinterpret_cast<const float*>(ws + L.xs);
+  A.sorted = reinterpret_cast<const int32_t*>(ws + L.sorted);
+  A.tiles = reinterpret_cast<const int4*>(ws + L.h);
+  A.n_tiles = reinterpret_cast<const int32_t*>(ws + L.n_tiles);
+  A.aq = reinterpret_cast<uint8_t*>(ws + L.aq);
+  A.as = reinterpret_cast<float*>(ws + L.as);
+  A.w = w13;  A.ws = s13;  A.w_es = es.w13;  A.s_es = es.s13;
+  A.top_k = top_k;  A.rows = 2 * inter;  A.G = hidden / 128;  A.inter = inter;
+  A.tiled = es.layout == MOE_LAYOUT_TILES;
+  A.ipt = inter / 128;
+  // Neighbouring tiles are mostly one expert's and share its weights in an
+  // XCD's L2; fewer than one run of four per XCD would leave XCDs idle.  Runs
+  // of 1 / 2 / 4 / 8 tiles, 256 experts, 4096 tokens: 482 / 412 / 393 / 390
+  // us; 2000 tokens of uneven popularity, runs of 4 / 8 / 16: 265 / 273 / 285;
+  // 16 experts, 100 tokens (17 tiles), 1 / 4: 40.6 / 43.0.
+  A.chunk = tiles >= 32 ? 4 : 1;
+  // Past the caches when the call reads about one tile of every expert and the
+  // experts don't fit the 256 MB last-level cache: 1021 tokens over 256 experts
+  // (805 MB) 203 -> 184 us, 300 over 64 of H 2560, I 256 (126 MB) 49 -> 56;
+  // 2000 over 256 (two tiles per expert) 267 -> 272.  Row-major loads use each
+  // line twice, and the down projection measured slower past the caches (1021
+  // tokens 64 -> 70 us).
+  A.stream = A.tiled && P < 48LL * n_experts &&
+             3LL * hidden * inter * n_experts > (256LL << 20);
+  int rc = launch_grouped_wide(A, true, max_tiles, s);
+  if (rc) return rc;
+  A.act = A.aq;  A.act_s = A.as;
+  A.w = w2;  A.ws = s2;  A.w_es = es.w2;  A.s_es = es.s2;
+  A.out = reinterpret_cast<float*>(ws + L.y);
+  A.rows = hidden;  A.G = inter / 128;
+  // two row blocks per item (4096 tokens, 1 / 2 / 4 blocks: 137 / 127 / 133
+  // us) while that leaves an item per CU
+  const int nblk = hidden / kWideDownRows;
+  A.blocks = nblk >= 2 && tiles * nblk >= 512 ? 2 : 1;
+  A.ipt = (nblk + A.blocks - 1) / A.blocks;
+  A.stream = 0;
+  return launch_grouped_wide(A, false, max_tiles, s);
+}
+
 // --------------------------------------------------------------- driver
 
 GroupedLayout grouped_layout(int32_t tokens, int32_t top_k, int32_t n_experts, int32_t hidden,
@@ -495,11 +546,19 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   int32_t* n_tiles = reinterpret_cast<int32_t*>(ws + L.n_tiles);
   const int64_t P = static_cast<int64_t>(tokens) * top_k;
   const int64_t max_tiles = (P + kTileTok - 1) / kTileTok + n_experts;
+  // (h holds the wide tiles' records: nothing else of that path uses it)
+  const bool wide = use_wide(P, n_experts, hidden);
   // the permutation and the activation rows' quantisation in one launch
   const QuantRowsJob quant{x, hidden, xq, xs, tokens};
-  int rc = launch_permute(ids, ids64, P, n_experts, counts, offsets, sorted, pos, s, tiles, n_tiles,
-                          kTileTok, &quant);
+  int rc = launch_permute(ids, ids64, P, n_experts, counts, offsets, sorted, pos, s,
+                          wide ? reinterpret_cast<int32_t*>(h) : tiles, n_tiles,
+                          wide ? kWideTile : kTileTok, &quant, wide);
   if (rc) return rc;
+  if (wide) {
+    rc = launch_wide(L, ws, P, top_k, w13, s13, w2, s2, es, n_experts, hidden, inter, s);
+    if (rc) return rc;
+    return launch_unpermute(y, pos, weights, wbf16, tokens, top_k, hidden, residual, out, s);
+  }
   StreamArgs gu{};
   gu.act = xq;  gu.act_s = xs;  gu.sorted = sorted;
   gu.counts = counts;  gu.offsets = offsets;  gu.tiles = tiles;  gu.n_tiles = n_tiles;

@@ -46,15 +46,43 @@ __device__ __forceinline__ void quant_row(const QuantRowsJob& q, int64_t t, int 
 // permute.hip
 // tiles (nullable): (expert, first segment row) of every tile_tokens rows of
 // every expert's segment, in expert order, and their count in *n_tiles.
+// wide_tiles: the records of grouped_wide.hip in `tiles` instead (int4).
 // quant (nullable): activation rows quantised by extra workgroups of the
 // same launch, two tokens each, beside the one that permutes.
 int launch_permute(const void* ids, int ids64, int64_t P, int32_t n_experts, int32_t* counts,
                    int32_t* offsets, int32_t* sorted_pairs, int32_t* pair_pos, hipStream_t s,
                    int32_t* tiles = nullptr, int32_t* n_tiles = nullptr, int32_t tile_tokens = 16,
-                   const QuantRowsJob* quant = nullptr);
+                   const QuantRowsJob* quant = nullptr, bool wide_tiles = false);
 int launch_unpermute(const float* y, const int32_t* pair_pos, const void* weights, int wbf16,
                      int32_t tokens, int32_t top_k, int32_t hidden, const uint16_t* residual,
                      uint16_t* out, hipStream_t s);
+
+// grouped_wide.hip: one projection of the grouped path over token tiles of
+// kWideTile rows (the tiles the permute launch listed).
+// A tile's record is (expert, first permuted row, rows of its expert from
+// there on, unused).
+constexpr int kWideTile = 64;
+constexpr int kWideDownRows = 256;   // rows of w2 per row block of a down item
+struct WideArgs {
+  const uint8_t* act;      // activation rows, e4m3, G*128 bytes each
+  const float* act_s;      // their per-128 scales, G per row
+  const int32_t* sorted;   // gate/up: permuted row -> token * top_k + k
+  const int4* tiles;       // tile records
+  const int32_t* n_tiles;
+  const uint8_t* w;        // [E][rows][G*128] e4m3, expert stride w_es bytes
+  const float* ws;         // [E][rows/128][G] f32, expert stride s_es floats
+  float* out;              // down: y [pairs][rows] f32, permuted order
+  uint8_t* aq;             // gate/up: SiLU(gate) * up, e4m3 [pairs][inter]
+  float* as;               // and its scales [pairs][inter / 128]
+  int64_t w_es, s_es;
+  int32_t top_k, rows, G, tiled, inter;
+  int32_t ipt;             // items per tile: inter / 128, or row blocks / blocks
+  int32_t blocks;          // down: row blocks per item
+  int32_t stream;          // read the weights past the caches
+  int32_t chunk;           // consecutive tiles per XCD turn
+  int32_t max_tiles;       // records that may be read (set by the launcher)
+};
+int launch_grouped_wide(const WideArgs& A, bool gate_up, int64_t max_tiles, hipStream_t s);
 
 // grouped.hip: workspace layout of the grouped path (byte offsets, 256-aligned)
 struct GroupedLayout {

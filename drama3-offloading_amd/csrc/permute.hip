@@ -78,11 +78,23 @@ __device__ __forceinline__ void wave_match_rank(int32_t e, int nbits, uint64_t b
   count = __popcll(m);
 }
 
+// Work tile n of the grouped kernels: rows m .. of the segment of expert e
+// (n_rows rows from permuted row `first`).
+__device__ __forceinline__ void put_tile(int32_t* tiles, int32_t n, int32_t e, int32_t first,
+                                         int32_t n_rows, int32_t m, int wide) {
+  if (wide) {
+    reinterpret_cast<int4*>(tiles)[n] = make_int4(e, first + m, n_rows - m, 0);
+  } else {
+    tiles[2 * n] = e;
+    tiles[2 * n + 1] = m;
+  }
+}
+
 __global__ __launch_bounds__(kPlaceThreads) void permute_kernel(
     const void* __restrict__ ids, int ids64, int64_t P, int32_t n_experts,
     int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ sorted_pairs,
     int32_t* __restrict__ pair_pos, int32_t* __restrict__ tiles, int32_t* __restrict__ n_tiles,
-    int32_t tile_tokens, QuantRowsJob quant) {
+    int32_t tile_tokens, int wide_tiles, QuantRowsJob quant) {
   __shared__ int32_t cursor[kPermMaxExperts];
   __shared__ uint64_t fields[kPermMaxExperts];
   __shared__ int32_t scratch[40];
@@ -149,6 +161,7 @@ __global__ __launch_bounds__(kPlaceThreads) void permute_kernel(
     // for every tile_tokens rows of every expert's segment, in expert order
     int32_t nt[kPlacePer];
     int32_t tsum = 0;
+    base -= sum;                   // back to the thread's first expert
 #pragma unroll
     for (int j = 0; j < kPlacePer; ++j) {
       nt[j] = (mine[j] + tile_tokens - 1) / tile_tokens;
@@ -159,10 +172,9 @@ __global__ __launch_bounds__(kPlaceThreads) void permute_kernel(
 #pragma unroll
     for (int j = 0; j < kPlacePer; ++j) {
       const int x = tid * kPlacePer + j;
-      for (int32_t i = 0; i < nt[j]; ++i) {
-        tiles[2 * (tbase + i)] = x;
-        tiles[2 * (tbase + i) + 1] = i * tile_tokens;
-      }
+      for (int32_t i = 0; i < nt[j]; ++i)
+        put_tile(tiles, tbase + i, x, base, mine[j], i * tile_tokens, wide_tiles);
+      base += mine[j];
       tbase += nt[j];
     }
     if (tid == 0) *n_tiles = ttotal;
@@ -236,7 +248,7 @@ __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
     const void* __restrict__ ids, int ids64, int64_t P, int32_t n_experts,
     int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ sorted_pairs,
     int32_t* __restrict__ pair_pos, int32_t* __restrict__ tiles, int32_t* __restrict__ n_tiles,
-    int32_t tile_tokens, QuantRowsJob quant) {
+    int32_t tile_tokens, int wide_tiles, QuantRowsJob quant) {
   __shared__ int32_t cursor[kFastExperts];
   __shared__ uint16_t wcount[kFastWaves * kFastExperts];   // [wave][expert]
   __shared__ int32_t scratch[40];
@@ -295,10 +307,8 @@ __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
     const int32_t nt = (mine + tile_tokens - 1) / tile_tokens;
     int32_t tbase;
     const int32_t ttotal = block_exclusive_scan<kFastWaves>(nt, scratch, &tbase);
-    for (int32_t i = 0; i < nt; ++i) {
-      tiles[2 * (tbase + i)] = tid;
-      tiles[2 * (tbase + i) + 1] = i * tile_tokens;
-    }
+    for (int32_t i = 0; i < nt; ++i)
+      put_tile(tiles, tbase + i, tid, base, mine, i * tile_tokens, wide_tiles);
     if (tid == 0) *n_tiles = ttotal;
   }
   __syncthreads();
@@ -477,7 +487,7 @@ __global__ __launch_bounds__(64) void gather_plan_kernel(
 int launch_permute(const void* ids, int ids64, int64_t P, int32_t n_experts, int32_t* counts,
                    int32_t* offsets, int32_t* sorted_pairs, int32_t* pair_pos, hipStream_t s,
                    int32_t* tiles, int32_t* n_tiles, int32_t tile_tokens,
-                   const QuantRowsJob* quant) {
+                   const QuantRowsJob* quant, bool wide_tiles) {
   static_assert(kPlaceThreads == 512, "two 256-thread token slices per quantising workgroup");
   static_assert(kFastThreads == 1024, "four 256-thread token slices per quantising workgroup");
   const QuantRowsJob q = quant ? *quant : QuantRowsJob{nullptr, 0, nullptr, nullptr, 0};
@@ -485,12 +495,12 @@ int launch_permute(const void* ids, int ids64, int64_t P, int32_t n_experts, int
     const unsigned grid = 1 + static_cast<unsigned>((q.tokens + 3) / 4);
     hipLaunchKernelGGL(permute_fast_kernel, dim3(grid), dim3(kFastThreads), 0, s, ids, ids64, P,
                        n_experts, counts, offsets, sorted_pairs, pair_pos, tiles, n_tiles,
-                       tile_tokens, q);
+                       tile_tokens, wide_tiles ? 1 : 0, q);
   } else {
     const unsigned grid = 1 + static_cast<unsigned>((q.tokens + 1) / 2);
     hipLaunchKernelGGL(permute_kernel, dim3(grid), dim3(kPlaceThreads), 0, s, ids, ids64, P,
                        n_experts, counts, offsets, sorted_pairs, pair_pos, tiles, n_tiles,
-                       tile_tokens, q);
+                       tile_tokens, wide_tiles ? 1 : 0, q);
   }
   return check_launch("moe_permute");
 }

@@ -175,3 +175,65 @@ def test_grouped_long_rows_match_oracle(lib, dev):
     err = omoe.max_rel_err(got.float().cpu().numpy(), want)
     print(f"grouped (H={H}, I={I}) max rel err vs W8A8 oracle {err:.2e}")
     assert err <= TOL
+
+
+def _device_experts(seed, E, H, I, dev):
+    """Random e4m3 weights and scales made on the device."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    def rnd(*s):
+        return (torch.randn(s, generator=g, device=dev) * 80).clamp_(-448, 448).to(
+            torch.float8_e4m3fn)
+
+    def sc(*s):
+        return torch.rand(s, generator=g, device=dev) * 1e-4 + 1e-4
+
+    w13 = torch.cat([rnd(1, 2 * I, H) for _ in range(E)])
+    w2 = torch.cat([rnd(1, H, I) for _ in range(E)])
+    return (w13.view(torch.uint8), sc(E, 2 * I // 128, H // 128), w2.view(torch.uint8),
+            sc(E, H // 128, I // 128))
+
+
+@pytest.mark.parametrize("T,E,K,H,I", [
+    (18, 1, 1, 256, 128),        # the fewest rows of the wide tiles, one K-block of each projection
+    (64, 1, 1, 2048, 512), (65, 1, 1, 512, 256), (129, 1, 1, 1024, 512),   # around whole tiles
+    (100, 5, 3, 768, 384),       # a row block to spare, windows that end inside K
+    (300, 16, 8, 2048, 512), (90, 4, 4, 4096, 1152),      # three windows of down
+    (40, 6, 4, 8192, 2048),      # the largest expert; weights read past the caches
+])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_wide_tiles_equal_gemv(lib, dev, T, E, K, H, I, tiled):
+    """Many rows per expert: token tiles of 64 rows, bit-identical to the
+    per-pair GEMV for full, ragged and single-row column tiles, an expert
+    without rows and picks of no expert (their tokens are NaN)."""
+    from hostpool import RecordLayout
+    import hipfetch
+    devt = _device_experts(T + E, E, H, I, dev)
+    rng = np.random.default_rng(T)
+    ids = np.stack([rng.permutation(E)[:K] for _ in range(T)])
+    if E > 4:
+        ids[:, 0] = np.where(rng.random(T) < 0.6, 0, ids[:, 0])    # a crowded expert
+        ids[ids == E - 1] = 1                                      # one nobody picks
+    if T > 64 and E > 1:
+        ids[3, 0], ids[T - 1, K - 1] = -1, E
+    ids = torch.from_numpy(ids).to(dev)
+    w = torch.rand((T, K), generator=torch.Generator().manual_seed(T)).to(dev)
+    g = torch.Generator(device=dev).manual_seed(T)
+    x = torch.randn((T, H), generator=g, device=dev).to(torch.bfloat16)
+    if tiled:
+        lay = RecordLayout(H, I)
+        devt = lay.views(torch.cat([lay.pack(*(t[e:e + 1] for t in devt)) for e in range(E)]))
+    code = hipfetch.LAYOUT_TILES if tiled else hipfetch.LAYOUT_ROWS
+    say(f"wide tiles: T={T} E={E} K={K} H={H} I={I} tiled={tiled}")
+    outs = []
+    for mode in (1, 2):
+        out = torch.full((T + 1, H), 7.0, dtype=torch.bfloat16, device=dev)
+        ws = torch.empty(lib.fp8_moe_workspace(T, K, E, H, I), dtype=torch.uint8, device=dev)
+        lib.fp8_moe_forward(x, ids, w, devt[0].view(torch.float8_e4m3fn), devt[1],
+                            devt[2].view(torch.float8_e4m3fn), devt[3], out[:T], ws, mode=mode,
+                            residual=x, layout=code)
+        torch.cuda.synchronize()
+        assert bool((out[T] == 7).all())
+        outs.append(out[:T].view(torch.int16))
+    assert torch.equal(*outs)
+    bad = torch.isnan(outs[0].view(torch.bfloat16)).any(1).nonzero().view(-1).tolist()
+    assert bad == ([3, T - 1] if T > 64 and E > 1 else [])
