@@ -19,6 +19,9 @@ struct SharedRefs {
   uint16_t* act;         // [T, Is] bf16 scratch
   float* sig;            // [T] scratch
 };
+// How the launches carry it: not at all, on the vector units (its rows one
+// after another per token), on the matrix cores (kSharedMmaFrom tokens on).
+constexpr int kSharedNone = 0, kSharedGemv = 1, kSharedMma = 2;
 constexpr int kSharedJPW = 2;   // shared intermediate rows (gate + up) per kernel-1 wave
 
 // A slot table's next state, staged by the launch that resolved the call

@@ -126,13 +126,6 @@ __global__ __launch_bounds__(64 * kLinearWaves) void linear_bf16_kernel(
 // order differs from the one-token kernel's (the matrix cores add inside
 // each MFMA), so the outputs agree with the float64 product to within one
 // bf16 step, as that kernel's do.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ v4f mfma_bf16_16x16x32(u32x4 a, u32x4 b, v4f c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
 constexpr int kLinMmaWaves = 8;         // K slices per workgroup
 constexpr int kLinMmaChunks = 4;        // 64-wide K chunks per wave in flight
 constexpr int kLinMmaMaxTokens = 128;

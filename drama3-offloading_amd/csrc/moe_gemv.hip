@@ -153,7 +153,7 @@ constexpr int kGateUpChunk = 8;                  // K-blocks in flight per lane
 // launch.
 // The logits' round trip and the top-k take the place of the id load ahead
 // of the weight loads, and the top-k needs no launch of its own.
-template <bool SHARED, int TOPK>
+template <int SHARED, int TOPK>
 __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
     const uint16_t* __restrict__ x, const void* __restrict__ ids, int ids64, int32_t top_k,
     const uint8_t* __restrict__ w13, const float* __restrict__ s13, int64_t w13_es,
@@ -167,7 +167,17 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
   __shared__ __align__(16) float upsum[16];
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  if (SHARED && blockIdx.y >= static_cast<unsigned>(tokens * top_k)) {
+  if (SHARED == kSharedMma && blockIdx.y >= static_cast<unsigned>(tokens * top_k)) {
+    // one tile of the shared expert's gate/up: 8 columns, or the sigmoid gate
+    // row, of all tokens, with the parts of K and the sums of moe_shared_gate_up
+    __shared__ float mma_part[SHARED == kSharedMma ? kSharedPartFloats<1, 1, 8> : 1];
+    const int j = ((blockIdx.y - tokens * top_k) * gridDim.x + blockIdx.x) * 8;
+    if (j > sh.inter) return;                    // the whole workgroup
+    shared_gate_up_tile<1, 1, 8, 2, kGateUpWaves>(x, sh.wg, sh.wu, sh.wsg, tokens, hidden, sh.inter,
+                                                  sh.act, sh.sig, j, 0, mma_part);
+    return;
+  }
+  if (SHARED == kSharedGemv && blockIdx.y >= static_cast<unsigned>(tokens * top_k)) {
     // shared expert rows j0, j0 + 1 (gate and up each; j == Is is the sigmoid gate row)
     const int j0 =
         (((blockIdx.y - tokens * top_k) * gridDim.x + blockIdx.x) * kGateUpWaves + wave) *
@@ -379,6 +389,7 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
 // took 5.3-5.4 us, and 4.9 with both replaced by a plain byte copy.
 constexpr int kDownChunk = 4;   // K-blocks of w2 in flight per lane (inter 512 = one chunk)
 constexpr int kDownRows = 8;    // output rows per workgroup
+constexpr int kSharedDownChunks = 4;   // 64-wide chunks of the shared expert's rows in flight
 
 // The down launch's extra workgroup: the staged table copied into the table.
 __device__ __forceinline__ void commit_table(const TableCommit& cm) {
@@ -391,7 +402,7 @@ __device__ __forceinline__ void commit_table(const TableCommit& cm) {
   if (threadIdx.x == 0) *cm.step_dst = *cm.step_src;
 }
 
-template <bool SHARED>
+template <int SHARED>
 __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
     const float* __restrict__ act, const void* __restrict__ ids, int ids64,
     const void* __restrict__ weights, int wbf16, int32_t top_k, const uint8_t* __restrict__ w2,
@@ -407,7 +418,7 @@ __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
   extern __shared__ __align__(16) uint8_t down_smem[];
   __shared__ __align__(16) float part[kMaxK + 1][kDownRows];   // [kMaxK]: discarded quadrants
   __shared__ float wpart[kMaxK];
-  __shared__ float spart[SHARED ? kDownRows : 1];
+  __shared__ __align__(16) float spart[SHARED ? kDownRows : 1];
   PHASE_MARKS_DECL;
   PHASE_MARK(0);                       // start
   const int wave = threadIdx.x >> 6;
@@ -417,7 +428,21 @@ __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
   const int kwaves = (top_k + 1) >> 1;
   uint8_t* const aq = down_smem;
   float* const as_ = reinterpret_cast<float*>(down_smem + 2 * kwaves * inter);
-  if (SHARED && wave == kwaves) {
+  if (SHARED == kSharedMma && wave == kwaves) {
+    // the shared expert's 8 down rows of this workgroup, token t: the tile of
+    // moe_shared_down with its rows twice and every column token t
+    const int i = lane & 15, sq = lane >> 4;
+    const uint16_t* const rows[1] = {sh.wd + static_cast<int64_t>(c0 + (i & 7)) * sh.inter + 16 * sq};
+    const uint16_t* const toks[1] = {sh.act + static_cast<int64_t>(t) * sh.inter + 16 * sq};
+    v4f sacc[1][1] = {{{0.f, 0.f, 0.f, 0.f}}};
+    shared_down_chain<1, kSharedDownChunks>(rows, toks, sh.inter >> 6, sacc);
+    if (i == 0 && sq < 2)
+      *reinterpret_cast<float4*>(&spart[4 * sq]) =
+          make_float4(sacc[0][0][0], sacc[0][0][1], sacc[0][0][2], sacc[0][0][3]);
+    __syncthreads();   // pairs with the routed waves' barrier: threads 0..7 then
+    return;            // combine, spart included
+  }
+  if (SHARED == kSharedGemv && wave == kwaves) {
     // the shared expert's 8 down rows of this workgroup, token t
     const uint16_t* rows[kDownRows];
 #pragma unroll
@@ -611,7 +636,6 @@ __global__ __launch_bounds__(64 * (kMaxK / 2 + 1)) void down_gemv_kernel(
 // those indices, so the four MFMAs cover the block once.  Grids, waves, the
 // weights' loads, the in-order K-block chains and the k-order combine are
 // the e4m3 kernels'.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // 8 e4m3 bytes (two words, lowest byte first) -> 8 bf16 in the same order.
@@ -900,7 +924,8 @@ static unsigned gateup_a16_lds(int32_t hidden) {
   return static_cast<unsigned>(hidden * 2 + kGateUpTiles * (hidden >> 7) * 17 * 4);
 }
 
-// The two decode launches; `sh` (nullable) carries the shared expert along.
+// The two decode launches; `sh` (nullable) carries the shared expert along,
+// on the vector units or the matrix cores as its own kernels do at this many tokens.
 // The router of up to 16 tokens in front of the GEMV launches: its logits launch
 // (gate weight, bias, logit rounding, the logits buffer), then the top-k
 // made inside the gate/up launch (gateup_gemv_kernel's TOPK), which writes
@@ -922,11 +947,20 @@ static int launch_gemv(const uint16_t* x, const void* ids, int ids64, const void
                        const SharedRefs* sh, hipStream_t s, const RouterTopK* rt = nullptr) {
   const int64_t pairs = static_cast<int64_t>(tokens) * top_k;
   const unsigned gx = static_cast<unsigned>((2 * inter) / 16);
-  if (sh) {
+  const bool sh_mma = sh && tokens >= kSharedMmaFrom;
+  if (sh_mma) {
+    // extra rows of workgroups for the shared expert's Is / 8 + 1 tiles
+    const unsigned per_y = gx / kGateUpTiles;
+    const unsigned sy = static_cast<unsigned>((sh->inter / 8 + 1 + per_y - 1) / per_y);
+    hipLaunchKernelGGL((gateup_gemv_kernel<kSharedMma, 0>), dim3(gx / kGateUpTiles, pairs + sy),
+                       dim3(64 * kGateUpWaves), 0, s, x, ids,
+                       ids64, top_k, w13, s13, es.w13, es.s13, static_cast<int>(es.layout),
+                       n_experts, hidden, inter, h, tokens, *sh, nullptr, nullptr);
+  } else if (sh) {
     // extra rows of workgroups for the shared expert's Is + 1 rows (the last: sigmoid gate)
     const unsigned per_y = kSharedJPW * (gx / kGateUpTiles) * kGateUpWaves;
     const unsigned sy = static_cast<unsigned>((sh->inter + 1 + per_y - 1) / per_y);
-    hipLaunchKernelGGL((gateup_gemv_kernel<true, 0>), dim3(gx / kGateUpTiles, pairs + sy),
+    hipLaunchKernelGGL((gateup_gemv_kernel<kSharedGemv, 0>), dim3(gx / kGateUpTiles, pairs + sy),
                        dim3(64 * kGateUpWaves), 0, s, x, ids,
                        ids64, top_k, w13, s13, es.w13, es.s13, static_cast<int>(es.layout),
                        n_experts, hidden, inter, h, tokens, *sh, nullptr, nullptr);
@@ -937,17 +971,17 @@ static int launch_gemv(const uint16_t* x, const void* ids, int ids64, const void
     weights = rt->weights;
     wbf16 = 0;
     if (n_experts <= 256)
-      hipLaunchKernelGGL((gateup_gemv_kernel<false, 4>), dim3(gx / kGateUpTiles, pairs),
+      hipLaunchKernelGGL((gateup_gemv_kernel<kSharedNone, 4>), dim3(gx / kGateUpTiles, pairs),
                          dim3(64 * kGateUpWaves), 0, s, x, ids, 0, top_k, w13, s13, es.w13,
                          es.s13, static_cast<int>(es.layout), n_experts, hidden, inter, h, tokens,
                          SharedRefs{}, rt->logits, rt->weights);
     else
-      hipLaunchKernelGGL((gateup_gemv_kernel<false, 16>), dim3(gx / kGateUpTiles, pairs),
+      hipLaunchKernelGGL((gateup_gemv_kernel<kSharedNone, 16>), dim3(gx / kGateUpTiles, pairs),
                          dim3(64 * kGateUpWaves), 0, s, x, ids, 0, top_k, w13, s13, es.w13,
                          es.s13, static_cast<int>(es.layout), n_experts, hidden, inter, h, tokens,
                          SharedRefs{}, rt->logits, rt->weights);
   } else {
-    hipLaunchKernelGGL((gateup_gemv_kernel<false, 0>), dim3(gx / kGateUpTiles, pairs),
+    hipLaunchKernelGGL((gateup_gemv_kernel<kSharedNone, 0>), dim3(gx / kGateUpTiles, pairs),
                        dim3(64 * kGateUpWaves), 0, s, x, ids, ids64,
                        top_k, w13, s13, es.w13, es.s13, static_cast<int>(es.layout), n_experts,
                        hidden, inter, h, tokens, SharedRefs{}, nullptr, nullptr);
@@ -955,13 +989,14 @@ static int launch_gemv(const uint16_t* x, const void* ids, int ids64, const void
   int rc = check_launch("moe_fp8_moe_forward(gate/up)");
   if (rc) return rc;
   if (sh) {
-    hipLaunchKernelGGL(down_gemv_kernel<true>, dim3(hidden / kDownRows, tokens),
+    const auto down = sh_mma ? down_gemv_kernel<kSharedMma> : down_gemv_kernel<kSharedGemv>;
+    hipLaunchKernelGGL(down, dim3(hidden / kDownRows, tokens),
                        dim3(64 * ((top_k + 1) / 2 + 1)),
                        down_lds(top_k, inter), s, h, ids, ids64, weights, wbf16, top_k, w2, s2,
                        es.w2, es.s2, static_cast<int>(es.layout), n_experts, hidden, inter, residual, out, *sh,
                        TableCommit{});
   } else {
-    hipLaunchKernelGGL(down_gemv_kernel<false>, dim3(hidden / kDownRows, tokens),
+    hipLaunchKernelGGL(down_gemv_kernel<kSharedNone>, dim3(hidden / kDownRows, tokens),
                        dim3(64 * ((top_k + 1) / 2)), down_lds(top_k, inter), s,
                        h, ids, ids64, weights, wbf16, top_k, w2, s2, es.w2, es.s2,
                        static_cast<int>(es.layout), n_experts, hidden, inter, residual, out,
@@ -999,12 +1034,12 @@ int launch_down_gemv(const float* act, const int32_t* slots, const void* weights
   const TableCommit cm = commit ? *commit : TableCommit{};
   const unsigned extra = commit ? 1u : 0u;
   if (sh) {
-    hipLaunchKernelGGL(down_gemv_kernel<true>, dim3(hidden / kDownRows + extra, tokens),
+    hipLaunchKernelGGL(down_gemv_kernel<kSharedGemv>, dim3(hidden / kDownRows + extra, tokens),
                        dim3(64 * ((top_k + 1) / 2 + 1)), down_lds(top_k, inter), s, act, slots, 0,
                        weights, wbf16, top_k, w2, s2, w2_es, s2_es, tiled, n_slots, hidden, inter, residual, out,
                        *sh, cm);
   } else {
-    hipLaunchKernelGGL(down_gemv_kernel<false>, dim3(hidden / kDownRows + extra, tokens),
+    hipLaunchKernelGGL(down_gemv_kernel<kSharedNone>, dim3(hidden / kDownRows + extra, tokens),
                        dim3(64 * ((top_k + 1) / 2)), down_lds(top_k, inter), s, act, slots, 0, weights,
                        wbf16, top_k, w2, s2, w2_es, s2_es, tiled, n_slots, hidden, inter, residual, out,
                        SharedRefs{}, cm);
@@ -1026,9 +1061,9 @@ using namespace moe;
 // launches up to 16 tokens.
 constexpr int32_t kGemvMaxTokens = 16;
 // The block call carries the shared expert in the GEMV launches up to this
-// many tokens (its gate/up workgroups take the tokens one after another);
-// beyond, the routed call is followed by the two shared-expert kernels.
-constexpr int32_t kCarrySharedMaxTokens = 2;
+// many tokens (one tile of its matrix-core form); beyond, the routed call is
+// followed by the two shared-expert kernels.
+constexpr int32_t kCarrySharedMaxTokens = 16;
 
 static bool use_grouped(int32_t tokens, int32_t hidden, int32_t mode) {
   if (mode == 1 || mode == 3) return false;

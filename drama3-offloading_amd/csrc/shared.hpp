@@ -102,6 +102,147 @@ __device__ __forceinline__ uint16_t shared_out(float dsum, float sig, bool has_r
   return f32_to_bf16(v);
 }
 
+// ------------------------------------------------------ on the matrix cores
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ v4f mfma_bf16_16x16x32(u32x4 a, u32x4 b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// One 64-wide K chunk of NR weight rows' tiles against TT token tiles: lane
+// (q, i) holds K 16q .. 16q + 15 of row i of each tile, two MFMAs a product.
+template <int NR, int TT>
+struct MmaChunk {
+  u32x4 a[NR][2], b[TT][2];
+  __device__ __forceinline__ void load(const uint16_t* const (&rows)[NR],
+                                       const uint16_t* const (&toks)[TT], int64_t o) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      b[t][0] = load16(toks[t] + o);
+      b[t][1] = load16(toks[t] + o + 8);
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      a[r][0] = load16(rows[r] + o);
+      a[r][1] = load16(rows[r] + o + 8);
+    }
+  }
+  // live false: a chunk past the end (its loads re-read the last one) adds nothing
+  __device__ __forceinline__ void fold(v4f (&acc)[NR][TT], bool live) {
+    const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const u32x4 av = live ? a[r][h] : z;
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+          acc[r][t] = mfma_bf16_16x16x32(av, live ? b[t][h] : z, acc[r][t]);
+      }
+    }
+  }
+};
+
+// Gate and up rows of NR * 8 intermediate columns against 16 * TT tokens: one
+// 16-row tile (NR 1) is 8 gate rows and the 8 up rows of the same columns,
+// two (NR 2) are 16 of each.  K is split W ways (part v is the 64-wide chunks
+// v, v + W, ...; WAVES waves take the parts in turn), U chunks in flight, and the
+// partial tiles are added in wave order through `lds` (kSharedPartFloats).
+// Columns from j0, tokens from t0; j0 == inter is the sigmoid gate row: all
+// rows of its tiles are that row.
+template <int NR, int TT, int W>
+constexpr int kSharedPartFloats = W * NR * TT * 16 * 17;
+template <int NR, int TT, int W, int U, int WAVES = W>
+__device__ __forceinline__ void shared_gate_up_tile(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ wg, const uint16_t* __restrict__ wu,
+    const uint16_t* __restrict__ wsg, int32_t tokens, int32_t hidden, int32_t inter,
+    uint16_t* __restrict__ act, float* __restrict__ sig, int j0, int t0, float* lds) {
+  constexpr int NJ = NR * 8;                      // columns per workgroup
+  float (*part)[NR][TT][16][17] = reinterpret_cast<float (*)[NR][TT][16][17]>(lds);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int i = lane & 15, q = lane >> 4;
+  const bool gate_row = j0 >= inter;
+  const uint16_t* rows[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const bool up = NR == 1 ? i >= 8 : r == 1;
+    const int j = j0 + (NR == 1 ? i & 7 : i);
+    rows[r] = (gate_row ? wsg : (up ? wu : wg) + static_cast<int64_t>(j) * hidden) + 16 * q;
+  }
+  const uint16_t* toks[TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+    toks[t] = x + static_cast<int64_t>(min(t0 + 16 * t + i, tokens - 1)) * hidden + 16 * q;
+  const int nchunk = hidden >> 6;                 // hidden % 128 == 0
+  for (int v = wave; v < W; v += WAVES) {
+    v4f acc[NR][TT];
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) acc[r][t] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int c0 = v; c0 < nchunk; c0 += W * U) {
+      MmaChunk<NR, TT> ch[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        ch[u].load(rows, toks, static_cast<int64_t>(min(c0 + u * W, nchunk - 1)) * 64);
+      __builtin_amdgcn_sched_barrier(0);          // every load is issued before the math below
+#pragma unroll
+      for (int u = 0; u < U; ++u) ch[u].fold(acc, c0 + u * W < nchunk);
+    }
+    // lane (q, i) holds rows 4q .. 4q + 3 of token column i
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) part[v][r][t][4 * q + k][i] = acc[r][t][k];
+  }
+  __syncthreads();
+  for (int o = threadIdx.x; o < TT * 16 * NJ; o += 64 * WAVES) {
+    const int rr = o % NJ, tc = (o / NJ) & 15, t = o / (16 * NJ);
+    const int ur = NR == 1 ? rr + 8 : rr;         // the up row of column rr in its tile
+    float g = part[0][0][t][rr][tc], u = part[0][NR - 1][t][ur][tc];
+#pragma unroll
+    for (int v = 1; v < W; ++v) {
+      g += part[v][0][t][rr][tc];
+      u += part[v][NR - 1][t][ur][tc];
+    }
+    const int tok = t0 + 16 * t + tc;
+    if (tok >= tokens) continue;
+    if (!gate_row)
+      act[static_cast<int64_t>(tok) * inter + j0 + rr] = shared_act(g, u);
+    else if (rr == 0)
+      sig[tok] = shared_sig(g);
+  }
+}
+
+// The down products of 16 rows and 16 * TT tokens: one chain over all of K, U
+// 64-wide chunks in flight (U changes only the load schedule).
+template <int TT, int U>
+__device__ __forceinline__ void shared_down_chain(const uint16_t* const (&rows)[1],
+                                                  const uint16_t* const (&toks)[TT], int nchunk,
+                                                  v4f (&acc)[1][TT]) {
+  for (int c0 = 0; c0 < nchunk; c0 += U) {
+    MmaChunk<1, TT> ch[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      ch[u].load(rows, toks, static_cast<int64_t>(min(c0 + u, nchunk - 1)) * 64);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) ch[u].fold(acc, c0 + u < nchunk);
+  }
+}
+
+// Fewest tokens of the matrix-core form.  Both kernels, H 2048, Is 512, a
+// graph over 40 layers' weights on MI355X, GEMV form -> matrix cores (us per
+// call, gate/up + down): 3 tokens 5.2 + 6.6 -> 4.8 + 3.8, 4 tokens 5.6 + 7.6
+// -> 5.0 + 3.8, 16 tokens 15.2 + 23.4 -> 5.9 + 3.9, 512 tokens 389 + 640 ->
+// 22.6 + 16.3.  One or two tokens stay on the GEMV form, whose sums the
+// decode launches that carry the shared expert reproduce.
+constexpr int kSharedMmaFrom = 3;
+
 // Launchers of the standalone shared-expert kernels (shared.hip).
 int launch_shared_gate_up(const uint16_t* x, const uint16_t* wg, const uint16_t* wu,
                           const uint16_t* wsg, int32_t tokens, int32_t hidden, int32_t inter,

@@ -98,7 +98,7 @@ def _routed_experts(seed, E, H, I, dev):
 
 
 @pytest.mark.parametrize("T,K,mode", [(1, 8, 0), (2, 8, 0), (1, 15, 0), (1, 16, 0), (5, 8, 0),
-                                      (3, 8, 1), (1, 8, 2)])
+                                      (3, 8, 1), (1, 8, 2), (16, 6, 0), (17, 8, 1), (9, 15, 0)])
 def test_block_forward_equals_composition(lib, dev, T, K, mode):
     """moe_fp8_moe_block_forward (the shared expert carried by the decode
     launches when T <= 2) against the composition of the three
