@@ -552,7 +552,8 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   const QuantRowsJob quant{x, hidden, xq, xs, tokens};
   int rc = launch_permute(ids, ids64, P, n_experts, counts, offsets, sorted, pos, s,
                           wide ? reinterpret_cast<int32_t*>(h) : tiles, n_tiles,
-                          wide ? kWideTile : kTileTok, &quant, wide);
+                          wide ? kWideTile : kTileTok, &quant, wide,
+                          reinterpret_cast<int32_t*>(y));   // y is free until the down launch
   if (rc) return rc;
   if (wide) {
     rc = launch_wide(L, ws, P, top_k, w13, s13, w2, s2, es, n_experts, hidden, inter, s);

@@ -47,12 +47,15 @@ __device__ __forceinline__ void quant_row(const QuantRowsJob& q, int64_t t, int 
 // tiles (nullable): (expert, first segment row) of every tile_tokens rows of
 // every expert's segment, in expert order, and their count in *n_tiles.
 // wide_tiles: the records of grouped_wide.hip in `tiles` instead (int4).
+// hist (nullable): scratch of ceil(P / 4096) * n_experts counts, with which a
+// call of several placement passes runs them side by side.
 // quant (nullable): activation rows quantised by extra workgroups of the
 // same launch, two tokens each, beside the one that permutes.
 int launch_permute(const void* ids, int ids64, int64_t P, int32_t n_experts, int32_t* counts,
                    int32_t* offsets, int32_t* sorted_pairs, int32_t* pair_pos, hipStream_t s,
                    int32_t* tiles = nullptr, int32_t* n_tiles = nullptr, int32_t tile_tokens = 16,
-                   const QuantRowsJob* quant = nullptr, bool wide_tiles = false);
+                   const QuantRowsJob* quant = nullptr, bool wide_tiles = false,
+                   int32_t* hist = nullptr);
 int launch_unpermute(const float* y, const int32_t* pair_pos, const void* weights, int wbf16,
                      int32_t tokens, int32_t top_k, int32_t hidden, const uint16_t* residual,
                      uint16_t* out, hipStream_t s);

@@ -244,16 +244,24 @@ constexpr int kFastRounds = 4;
 constexpr int kFastPass = kFastThreads * kFastRounds;   // pairs per placement pass
 constexpr int kFastExperts = 1024;                      // one thread per expert
 
+//
+// SPLIT: one workgroup per pass, for calls of several passes that have the
+// passes' counts already (hist [passes][E], permute_count_kernel): each
+// workgroup adds them up itself, workgroup 0 writes the counts, offsets and
+// tiles.  The passes of the one workgroup ran one after another, 7 us each:
+// the launch took 58 us at 4096 tokens top-8 (8 passes) and 16 at 1021 (2), the
+// two take 10.8 + 11.6 and 4.9 + 8.7.
+template <bool SPLIT>
 __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
     const void* __restrict__ ids, int ids64, int64_t P, int32_t n_experts,
     int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ sorted_pairs,
     int32_t* __restrict__ pair_pos, int32_t* __restrict__ tiles, int32_t* __restrict__ n_tiles,
-    int32_t tile_tokens, int wide_tiles, QuantRowsJob quant) {
+    int32_t tile_tokens, int wide_tiles, const int32_t* __restrict__ hist, QuantRowsJob quant) {
   __shared__ int32_t cursor[kFastExperts];
   __shared__ uint16_t wcount[kFastWaves * kFastExperts];   // [wave][expert]
   __shared__ int32_t scratch[40];
   const int tid = threadIdx.x;
-  if (blockIdx.x > 0) {
+  if (!SPLIT && blockIdx.x > 0) {
     // the activation rows, four tokens per workgroup (a 256-thread quarter
     // each, whole waves), beside workgroup 0's permutation; no barrier here
     const int64_t t = 4 * static_cast<int64_t>(blockIdx.x - 1) + (tid >> 8);
@@ -272,36 +280,54 @@ __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
       e[j] = p < P ? ((v >= 0 && v < E) ? v : -1) : -2;
     }
   };
+  const int64_t p_first = SPLIT ? static_cast<int64_t>(blockIdx.x) * kFastPass : 0;
+  const int64_t p_end = SPLIT ? min(P, p_first + kFastPass) : P;
+  const bool writer = !SPLIT || blockIdx.x == 0;   // of what is the call's, not the pass's
   int32_t held[kFastRounds];
 #pragma unroll
   for (int j = 0; j < kFastRounds; ++j) held[j] = -2;
-  if (P > 0) load_pass(0, held);
+  if (P > 0) load_pass(p_first, held);
   if (tid < E) {
     cursor[tid] = 0;
 #pragma unroll
     for (int w = 0; w < kFastWaves; ++w) wcount[w * kFastExperts + tid] = 0;
   }
   __syncthreads();
-  // histogram (LDS atomics; the counts do not depend on the order)
+  int32_t mine = 0, before = 0;    // expert tid's pairs, and those of earlier passes
+  if constexpr (SPLIT) {
+    const int n_pass = static_cast<int>(gridDim.x);
+    if (tid < E) {
+#pragma unroll 8
+      for (int c = 0; c < n_pass; ++c) {
+        const int32_t v = hist[static_cast<int64_t>(c) * E + tid];
+        mine += v;
+        before += c < static_cast<int>(blockIdx.x) ? v : 0;
+      }
+    }
+  } else {
+    // histogram (LDS atomics; the counts do not depend on the order)
 #pragma unroll
-  for (int j = 0; j < kFastRounds; ++j)
-    if (held[j] >= 0) atomicAdd(&cursor[held[j]], 1);
-  for (int64_t p = kFastPass + tid; p < P; p += kFastThreads) {
-    const int32_t v = read_id(ids, ids64, p);
-    if (v >= 0 && v < E) atomicAdd(&cursor[v], 1);
+    for (int j = 0; j < kFastRounds; ++j)
+      if (held[j] >= 0) atomicAdd(&cursor[held[j]], 1);
+    for (int64_t p = kFastPass + tid; p < P; p += kFastThreads) {
+      const int32_t v = read_id(ids, ids64, p);
+      if (v >= 0 && v < E) atomicAdd(&cursor[v], 1);
+    }
+    __syncthreads();
+    mine = tid < E ? cursor[tid] : 0;
   }
-  __syncthreads();
   // thread t owns expert t: counts, offsets, and the placement cursor
-  const int32_t mine = tid < E ? cursor[tid] : 0;
   int32_t base;
   const int32_t total = block_exclusive_scan<kFastWaves>(mine, scratch, &base);
   if (tid < E) {
-    counts[tid] = mine;
-    offsets[tid] = base;
-    cursor[tid] = base;
+    if (writer) {
+      counts[tid] = mine;
+      offsets[tid] = base;
+    }
+    cursor[tid] = base + before;
   }
-  if (tid == 0) offsets[E] = total;
-  if (tiles) {
+  if (tid == 0 && writer) offsets[E] = total;
+  if (tiles && writer) {
     // work tiles of the grouped kernels: (expert, first row of the segment)
     // for every tile_tokens rows of every expert's segment, in expert order
     const int32_t nt = (mine + tile_tokens - 1) / tile_tokens;
@@ -315,8 +341,8 @@ __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
   const uint64_t below_lane = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const int nbits = E > 1 ? 32 - __clz(E - 1) : 0;
   uint16_t* wc = wcount + wave * kFastExperts;
-  for (int64_t c0 = 0; c0 < P; c0 += kFastPass) {
-    if (c0 > 0) load_pass(c0, held);
+  for (int64_t c0 = p_first; c0 < p_end; c0 += kFastPass) {
+    if (c0 > p_first) load_pass(c0, held);
     // rank of each pair among its wave's pairs of the same expert
     int32_t rank[kFastRounds];
 #pragma unroll
@@ -363,6 +389,35 @@ __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
     }
     __syncthreads();
   }
+}
+
+// The expert counts of every placement pass, hist [n_pass][E], beside the
+// activation rows (four tokens per workgroup, as above).
+__global__ __launch_bounds__(kFastThreads) void permute_count_kernel(
+    const void* __restrict__ ids, int ids64, int64_t P, int32_t n_experts, int32_t n_pass,
+    int32_t* __restrict__ hist, QuantRowsJob quant) {
+  __shared__ int32_t cnt[kFastExperts];
+  const int tid = threadIdx.x;
+  const int c = static_cast<int>(blockIdx.x);
+  if (c >= n_pass) {
+    const int64_t t = 4 * static_cast<int64_t>(c - n_pass) + (tid >> 8);
+    if (t < quant.tokens) quant_row(quant, t, tid & 255);
+    return;
+  }
+  int32_t v[kFastRounds];
+#pragma unroll
+  for (int j = 0; j < kFastRounds; ++j) {
+    const int64_t p = static_cast<int64_t>(c) * kFastPass + j * kFastThreads + tid;
+    v[j] = read_id(ids, ids64, p < P ? p : P - 1);
+    if (p >= P) v[j] = -1;
+  }
+  if (tid < n_experts) cnt[tid] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kFastRounds; ++j)
+    if (v[j] >= 0 && v[j] < n_experts) atomicAdd(&cnt[v[j]], 1);
+  __syncthreads();
+  if (tid < n_experts) hist[static_cast<int64_t>(c) * n_experts + tid] = cnt[tid];
 }
 
 __global__ __launch_bounds__(kPermThreads) void unique_inverse_kernel(
@@ -487,15 +542,27 @@ __global__ __launch_bounds__(64) void gather_plan_kernel(
 int launch_permute(const void* ids, int ids64, int64_t P, int32_t n_experts, int32_t* counts,
                    int32_t* offsets, int32_t* sorted_pairs, int32_t* pair_pos, hipStream_t s,
                    int32_t* tiles, int32_t* n_tiles, int32_t tile_tokens,
-                   const QuantRowsJob* quant, bool wide_tiles) {
+                   const QuantRowsJob* quant, bool wide_tiles, int32_t* hist) {
   static_assert(kPlaceThreads == 512, "two 256-thread token slices per quantising workgroup");
   static_assert(kFastThreads == 1024, "four 256-thread token slices per quantising workgroup");
   const QuantRowsJob q = quant ? *quant : QuantRowsJob{nullptr, 0, nullptr, nullptr, 0};
-  if (n_experts <= kFastExperts) {
+  const int64_t n_pass = (P + kFastPass - 1) / kFastPass;
+  if (n_experts <= kFastExperts && hist && n_pass > 1) {
+    hipLaunchKernelGGL(permute_count_kernel, dim3(static_cast<unsigned>(n_pass + (q.tokens + 3) / 4)),
+                       dim3(kFastThreads), 0, s, ids, ids64, P, n_experts,
+                       static_cast<int32_t>(n_pass), hist, q);
+    const int rc = check_launch("moe_permute(count)");
+    if (rc) return rc;
+    hipLaunchKernelGGL(permute_fast_kernel<true>, dim3(static_cast<unsigned>(n_pass)),
+                       dim3(kFastThreads), 0, s, ids, ids64, P, n_experts, counts, offsets,
+                       sorted_pairs, pair_pos, tiles, n_tiles, tile_tokens, wide_tiles ? 1 : 0,
+                       hist, q);
+  } else if (n_experts <= kFastExperts) {
     const unsigned grid = 1 + static_cast<unsigned>((q.tokens + 3) / 4);
-    hipLaunchKernelGGL(permute_fast_kernel, dim3(grid), dim3(kFastThreads), 0, s, ids, ids64, P,
+    hipLaunchKernelGGL(permute_fast_kernel<false>, dim3(grid), dim3(kFastThreads), 0, s, ids, ids64, P,
                        n_experts, counts, offsets, sorted_pairs, pair_pos, tiles, n_tiles,
-                       tile_tokens, wide_tiles ? 1 : 0, q);
+                       tile_tokens, wide_tiles ? 1 : 0,
+                       nullptr, q);
   } else {
     const unsigned grid = 1 + static_cast<unsigned>((q.tokens + 1) / 2);
     hipLaunchKernelGGL(permute_kernel, dim3(grid), dim3(kPlaceThreads), 0, s, ids, ids64, P,

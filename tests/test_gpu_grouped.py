@@ -199,10 +199,12 @@ def _device_experts(seed, E, H, I, dev):
     (100, 5, 3, 768, 384),       # a row block to spare, windows that end inside K
     (300, 16, 8, 2048, 512), (90, 4, 4, 4096, 1152),      # three windows of down
     (40, 6, 4, 8192, 2048),      # the largest expert; weights read past the caches
+    # several placement passes: the last of one pair, wide and streamed tiles, 1000 experts
+    (4097, 2, 1, 256, 128), (1100, 300, 8, 128, 128), (1300, 1000, 7, 256, 128),
 ])
 @pytest.mark.parametrize("tiled", [False, True])
 def test_wide_tiles_equal_gemv(lib, dev, T, E, K, H, I, tiled):
-    """Many rows per expert: token tiles of 64 rows, bit-identical to the
+    """Many rows per expert or many pairs: token tiles of 64 rows, bit-identical to the
     per-pair GEMV for full, ragged and single-row column tiles, an expert
     without rows and picks of no expert (their tokens are NaN)."""
     from hostpool import RecordLayout
