@@ -175,10 +175,10 @@ __global__ __launch_bounds__(64 * kLogitWaves) void router_logits_kernel(
   if (ticket && e_raw == 0 && blockIdx.y == 0 && lane == 0) *ticket = 0;
 }
 
-// Many tokens: the logits on the float64 matrix cores.  A workgroup takes 16
-// experts x 16 tokens; its kLogitMmaWaves waves split K, wave v taking the
-// 32-wide chunks v, v + kLogitMmaWaves, ...  Lane (q, i) = (lane / 16, lane %
-// 16) loads 16 bytes of expert i's gate row and of token i's row, K 8q ..
+// Many tokens: the logits on the float64 matrix cores.  A workgroup takes TE x
+// TT tiles of 16 experts x 16 tokens; its W waves split K, wave v taking the
+// 32-wide chunks v, v + W, ...  Lane (q, i) = (lane / 16, lane % 16) loads 16
+// bytes of expert i's gate row and of token i's row of each tile, K 8q ..
 // 8q + 7 of a chunk, and each of its 8 bf16 pairs is one 16x16x4 float64
 // MFMA (the lane group q's K index of every MFMA), so every product of the
 // chunk is formed once, exact in float64.  The products are the vector
@@ -193,62 +193,107 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 // (moe_router_topk, 256 experts, H 2048, a graph over 40 gates): vector
 // 8.2 / 9.9 / 12.7 / 15.5 / 18.2 / 28.6 / 50.5 us at 16 / 32 / 64 / 96 /
 // 128 / 256 / 512 tokens, this form 12.0 up to 256 tokens and 19.2 at 512.
-constexpr int kLogitMmaWaves = 8;       // K slices per workgroup
-constexpr int kLogitMmaChunks = 8;      // 32-wide K chunks per wave in flight
+//
+// One tile per workgroup spreads a small call over the CUs, but converts two
+// operands to float64 per MFMA; several tiles share the conversions (one
+// operand per MFMA at 2 x 2).
 constexpr int kLogitMmaFrom = 64;       // tokens from which this form runs
+// Workgroups of 2 x 2 tiles from which they are used: two per CU.  MI355X, 256
+// experts, H 2048, one tile -> four (moe.route, with the top-k): 4096 tokens
+// (1024 workgroups) 111 -> 86 us; 1500 (376: one CU in two has two) 47.0 ->
+// 48.6; 2 x 4 tiles 85 and 49, 4 x 4 162.  The float64 MFMAs alone are 55 us at
+// 4096 tokens.
+constexpr int kLogitMmaBigFrom = 512;
 
 __device__ __forceinline__ double bf16_elem(u32x4 v, int m) {
   const uint32_t w = m < 2 ? v.x : m < 4 ? v.y : m < 6 ? v.z : v.w;
   return static_cast<double>(__uint_as_float((m & 1) ? (w & 0xffff0000u) : (w << 16)));
 }
 
-__global__ __launch_bounds__(64 * kLogitMmaWaves) void router_logits_mma_kernel(
+template <int TE, int TT, int W, int U>
+__global__ __launch_bounds__(64 * W) void router_logits_mma_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias,
     int32_t tokens, int32_t hidden, int32_t n_experts, int bf16_logits,
     float* __restrict__ logits) {
-  __shared__ double part[kLogitMmaWaves][16][17];
+  // independent sums per tile: enough of them to keep MFMAs in flight
+  constexpr int NA = TE * TT >= 4 ? 1 : 4;
+  __shared__ double part[W][TE][TT][16][17];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i = lane & 15, q = lane >> 4;
-  const int e0 = static_cast<int>(blockIdx.x) * 16, t0 = static_cast<int>(blockIdx.y) * 16;
-  const uint16_t* wr = w + static_cast<int64_t>(min(e0 + i, n_experts - 1)) * hidden + 8 * q;
-  const uint16_t* xr = x + static_cast<int64_t>(min(t0 + i, tokens - 1)) * hidden + 8 * q;
+  const int e0 = static_cast<int>(blockIdx.x) * 16 * TE;
+  const int t0 = static_cast<int>(blockIdx.y) * 16 * TT;
+  const uint16_t* wr[TE];
+  const uint16_t* xr[TT];
+#pragma unroll
+  for (int a = 0; a < TE; ++a)
+    wr[a] = w + static_cast<int64_t>(min(e0 + 16 * a + i, n_experts - 1)) * hidden + 8 * q;
+#pragma unroll
+  for (int b = 0; b < TT; ++b)
+    xr[b] = x + static_cast<int64_t>(min(t0 + 16 * b + i, tokens - 1)) * hidden + 8 * q;
   const int nchunk = hidden >> 5;
-  v4d acc[4];
+  v4d acc[TE][TT][NA];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) acc[c] = v4d{0.0, 0.0, 0.0, 0.0};
-  for (int c0 = wave; c0 < nchunk; c0 += kLogitMmaWaves * kLogitMmaChunks) {
-    u32x4 a[kLogitMmaChunks], b[kLogitMmaChunks];
+  for (int a = 0; a < TE; ++a)
 #pragma unroll
-    for (int u = 0; u < kLogitMmaChunks; ++u) {
-      const int64_t o = static_cast<int64_t>(min(c0 + u * kLogitMmaWaves, nchunk - 1)) * 32;
-      a[u] = *reinterpret_cast<const u32x4*>(wr + o);
-      b[u] = *reinterpret_cast<const u32x4*>(xr + o);
+    for (int b = 0; b < TT; ++b)
+#pragma unroll
+      for (int c = 0; c < NA; ++c) acc[a][b][c] = v4d{0.0, 0.0, 0.0, 0.0};
+  for (int c0 = wave; c0 < nchunk; c0 += W * U) {
+    u32x4 wv[U][TE], xv[U][TT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t o = static_cast<int64_t>(min(c0 + u * W, nchunk - 1)) * 32;
+#pragma unroll
+      for (int a = 0; a < TE; ++a) wv[u][a] = *reinterpret_cast<const u32x4*>(wr[a] + o);
+#pragma unroll
+      for (int b = 0; b < TT; ++b) xv[u][b] = *reinterpret_cast<const u32x4*>(xr[b] + o);
     }
     __builtin_amdgcn_sched_barrier(0);   // every load above is issued before the math below
 #pragma unroll
-    for (int u = 0; u < kLogitMmaChunks; ++u) {
+    for (int u = 0; u < U; ++u) {
       // a chunk past the end re-read the last one: zeros (no branch)
-      const bool live = c0 + u * kLogitMmaWaves < nchunk;
+      const bool live = c0 + u * W < nchunk;
+      const u32x4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int a = 0; a < TE; ++a) wv[u][a] = live ? wv[u][a] : zero;
+#pragma unroll
+      for (int b = 0; b < TT; ++b) xv[u][b] = live ? xv[u][b] : zero;
 #pragma unroll
       for (int m = 0; m < 8; ++m) {
-        const double av = live ? bf16_elem(a[u], m) : 0.0;
-        const double bv = live ? bf16_elem(b[u], m) : 0.0;
-        acc[m & 3] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[m & 3], 0, 0, 0);
+        double bv[TT];
+#pragma unroll
+        for (int b = 0; b < TT; ++b) bv[b] = bf16_elem(xv[u][b], m);
+#pragma unroll
+        for (int a = 0; a < TE; ++a) {
+          const double av = bf16_elem(wv[u][a], m);
+#pragma unroll
+          for (int b = 0; b < TT; ++b)
+            acc[a][b][m % NA] =
+                __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv[b], acc[a][b][m % NA], 0, 0, 0);
+        }
       }
     }
   }
   // element r of lane (q, i) holds expert 4r + q of token column i (the
   // float64 MFMA's result layout)
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    part[wave][4 * r + q][i] = (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
-  __syncthreads();
-  if (threadIdx.x < 256) {
-    const int rr = threadIdx.x & 15, j = threadIdx.x >> 4;
-    double sum = part[0][rr][j];
+  for (int a = 0; a < TE; ++a)
 #pragma unroll
-    for (int v = 1; v < kLogitMmaWaves; ++v) sum += part[v][rr][j];
-    const int e = e0 + rr, t = t0 + j;
+    for (int b = 0; b < TT; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        double v = acc[a][b][0][r];
+        if constexpr (NA == 4)
+          v = (acc[a][b][0][r] + acc[a][b][1][r]) + (acc[a][b][2][r] + acc[a][b][3][r]);
+        part[wave][a][b][4 * r + q][i] = v;
+      }
+  __syncthreads();
+  for (int o = threadIdx.x; o < 256 * TE * TT; o += 64 * W) {
+    const int rr = o & 15, a = (o >> 4) % TE, j = ((o >> 4) / TE) & 15, b = (o >> 8) / TE;
+    double sum = part[0][a][b][rr][j];
+#pragma unroll
+    for (int v = 1; v < W; ++v) sum += part[v][a][b][rr][j];
+    const int e = e0 + 16 * a + rr, t = t0 + 16 * b + j;
     if (e < n_experts && t < tokens) {
       float l = bf16_logits ? bf16_of_f64(sum) : static_cast<float>(sum);
       if (bias) l += bias[e];
@@ -370,10 +415,16 @@ int launch_router_logits(const void* x, const void* w, const float* bias, int32_
   const dim3 grid((n_experts + kLogitWaves - 1) / kLogitWaves,
                   (tokens + kTokBlock - 1) / kTokBlock);
   if (tokens >= kLogitMmaFrom && hidden % 32 == 0) {
-    hipLaunchKernelGGL(router_logits_mma_kernel, dim3((n_experts + 15) / 16, (tokens + 15) / 16),
-                       dim3(64 * kLogitMmaWaves), 0, s, static_cast<const uint16_t*>(x),
-                       static_cast<const uint16_t*>(w), bias, tokens, hidden, n_experts,
-                       bf16_logits, logits);
+    const unsigned gx = (n_experts + 31) / 32, gy = (tokens + 31) / 32;
+    if (static_cast<int64_t>(gx) * gy >= kLogitMmaBigFrom)
+      hipLaunchKernelGGL((router_logits_mma_kernel<2, 2, 4, 4>), dim3(gx, gy), dim3(64 * 4), 0, s,
+                         static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias,
+                         tokens, hidden, n_experts, bf16_logits, logits);
+    else
+      hipLaunchKernelGGL((router_logits_mma_kernel<1, 1, 8, 8>),
+                         dim3((n_experts + 15) / 16, (tokens + 15) / 16), dim3(64 * 8), 0, s,
+                         static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias,
+                         tokens, hidden, n_experts, bf16_logits, logits);
   } else if (tokens == 1)
     hipLaunchKernelGGL(router_logits_kernel<1>, grid, dim3(64 * kLogitWaves), 0, s,
                        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias,

@@ -175,12 +175,13 @@ def test_route_resolve_equals_router_then_resolve(lib, dev, logit_dtype):
     assert int(step.item()) == int(stp)
 
 
-@pytest.mark.parametrize("E,H,T", [(320, 1056, 100), (256, 2048, 64), (40, 96, 65)])
+@pytest.mark.parametrize("E,H,T", [(320, 1056, 100), (256, 2048, 64), (40, 96, 65),
+                                   (330, 160, 1500), (40, 96, 8200), (256, 2048, 2050)])
 def test_router_logits_matrix_cores_equal_vector_kernel(lib, dev, E, H, T):
     """From 64 tokens the logits run on the float64 matrix cores: the same
     logits, ids and weights as the vector kernel (the same call cut into
     pieces of fewer than 64 tokens), with a bias, ragged expert and token
-    tiles, and the oracle's ids."""
+    tiles, one or 2 x 2 of them per workgroup, and the oracle's ids."""
     g = torch.Generator(device="cpu").manual_seed(E + H + T)
     x = torch.randn((T, H), generator=g).to(torch.bfloat16).to(dev)
     w = (torch.randn((E, H), generator=g) * 0.02).to(torch.bfloat16).to(dev)
