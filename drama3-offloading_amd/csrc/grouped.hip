@@ -1,7 +1,8 @@
 // Grouped W8A8 expert FFN for many tokens (prefill, batched decode): token
 // rows are permuted into per-expert segments (permute.hip), the segments are
-// cut into tiles of up to 32 rows, every expert's weights are read from HBM
-// once per tile, and the results are un-permuted with the routing weights.
+// cut into tiles of up to 32 rows (16 or 64 in calls of few or many rows per
+// expert), every expert's weights are read from HBM once per tile, and the
+// results are un-permuted with the routing weights.
 //
 //   permute:     the token -> expert grouping and the tile list, and in the
 //                same launch x [T, H] bf16 -> xq [T, H] e4m3, xs [T, H/128]
@@ -38,7 +39,7 @@ namespace moe {
 // ---------------------------------------------------- streamed expert GEMM
 //
 // One kernel computes both projections.  For the weight rows r of one expert
-// and the permuted rows pos of one of its tiles (up to 32 consecutive rows
+// and the permuted rows pos of one of its tiles (up to TT consecutive rows
 // of the expert's segment, listed by the permute kernel):
 //
 //   out[pos][r] = sum over K-blocks kb, in order, of
@@ -63,7 +64,7 @@ namespace moe {
 // fill the chip (pick_shape).
 
 constexpr int kTileTok = 32;          // permuted rows per tile (two MFMA column tiles)
-constexpr int kColTiles = kTileTok / 16;
+constexpr int kSmallTileTok = 16;     // the same for calls of few rows per expert
 constexpr int kWaves = 4;             // waves per workgroup
 constexpr int kRing = 16;             // K-block operands in flight per lane
 constexpr int kStageBlocks = 16;      // K-blocks of activations staged at a time
@@ -74,11 +75,10 @@ constexpr int kMinItems = 400;        // fewest work items worth a bigger GPW
 
 // LDS of one workgroup: the activation tile first (the direct loads address
 // it from offset 0), then the scales and the tile's token rows.
-constexpr int kLdsAct = kTileTok * kStageRowBytes;
-constexpr int kLdsActScale = kLdsAct;
-constexpr int kLdsWScale = kLdsActScale + 4 * kTileTok * kStageBlocks;
-constexpr int kLdsTok = kLdsWScale + 4 * kMaxScaleRows * kStageBlocks;
-constexpr int kLdsBytes = kLdsTok + 4 * kTileTok;
+constexpr int lds_act(int rows) { return rows * kStageRowBytes; }
+constexpr int lds_wscale(int rows) { return lds_act(rows) + 4 * rows * kStageBlocks; }
+constexpr int lds_tok(int rows) { return lds_wscale(rows) + 4 * kMaxScaleRows * kStageBlocks; }
+constexpr int lds_bytes(int rows) { return lds_tok(rows) + 4 * rows; }
 
 struct StreamArgs {
   const uint8_t* act;      // activation rows, e4m3, G*128 bytes each
@@ -114,16 +114,17 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // the same row sums, then quantize8_f32, so the codes are identical.
 constexpr int kGluPad = 4;            // LDS row padding (floats) of the epilogue tile
 
-template <int RING, int GPW, bool GATHER, bool GLU>
-__global__ __launch_bounds__(64 * kWaves) void grouped_stream_kernel(StreamArgs A) {
+template <int RING, int GPW, bool GATHER, bool GLU, int TT>
+__global__ __launch_bounds__(64 * kWaves, TT == kSmallTileTok ? 4 : 1) void grouped_stream_kernel(StreamArgs A) {
   static_assert(RING % GPW == 0 && RING <= kRing && GPW <= kMaxGPW, "ring slots per group");
   static_assert(!GLU || GPW >= 4, "the GLU form needs whole 128-column groups per item");
   constexpr int KPP = RING / GPW;                   // K-blocks per pass of the ring
-  __shared__ __align__(16) uint8_t smem[kLdsBytes];
+  constexpr int kColTiles = TT / 16;                // TT: permuted rows per tile
+  __shared__ __align__(16) uint8_t smem[lds_bytes(TT)];
   uint8_t* xt = smem;
-  float* xst = reinterpret_cast<float*>(smem + kLdsActScale);
-  float* wsc = reinterpret_cast<float*>(smem + kLdsWScale);
-  int32_t* tok = reinterpret_cast<int32_t*>(smem + kLdsTok);
+  float* xst = reinterpret_cast<float*>(smem + lds_act(TT));
+  float* wsc = reinterpret_cast<float*>(smem + lds_wscale(TT));
+  int32_t* tok = reinterpret_cast<int32_t*>(smem + lds_tok(TT));
 
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
@@ -143,7 +144,7 @@ __global__ __launch_bounds__(64 * kWaves) void grouped_stream_kernel(StreamArgs 
   const int32_t e = A.tiles[2 * tile];
   const int32_t m0 = A.tiles[2 * tile + 1];
   const int32_t seg = A.offsets[e] + m0;            // first permuted row of the tile
-  const int32_t ncols = min(kTileTok, A.counts[e] - m0);
+  const int32_t ncols = min(TT, A.counts[e] - m0);
   const int nct = (ncols + 15) >> 4;                // column tiles in use
   const int row0 = static_cast<int>(item % ipt) * (64 * GPW);
   // GLU: the item's columns c0..c0+32*GPW-1; waves 0-1 take their gate rows,
@@ -169,7 +170,7 @@ __global__ __launch_bounds__(64 * kWaves) void grouped_stream_kernel(StreamArgs 
 
   // token rows of the tile (gather form), issued before the weights
   int32_t tokv = 0;
-  if (GATHER && threadIdx.x < kTileTok)
+  if (GATHER && threadIdx.x < TT)
     tokv = A.sorted[seg + min(static_cast<int>(threadIdx.x), ncols - 1)] / A.top_k;
   __builtin_amdgcn_sched_barrier(0);
 
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(64 * kWaves) void grouped_stream_kernel(StreamArgs 
   }
   __builtin_amdgcn_sched_barrier(0);
 
-  if (GATHER && threadIdx.x < kTileTok) tok[threadIdx.x] = tokv;
+  if (GATHER && threadIdx.x < TT) tok[threadIdx.x] = tokv;
   __syncthreads();
 
   auto act_row = [&](int r) -> int64_t {
@@ -293,7 +294,7 @@ __global__ __launch_bounds__(64 * kWaves) void grouped_stream_kernel(StreamArgs 
     // free once every wave is past its last K-block)
     constexpr int kCols = 32 * GPW;                 // columns of the item
     constexpr int kStride = kCols + kGluPad;
-    static_assert(2 * kTileTok * kStride * 4 <= kLdsBytes, "GLU epilogue tile fits the LDS");
+    static_assert(2 * TT * kStride * 4 <= lds_bytes(TT), "GLU epilogue tile fits the LDS");
     float* ep = reinterpret_cast<float*>(smem);
     __syncthreads();
     const int half = wave >> 1;
@@ -303,7 +304,7 @@ __global__ __launch_bounds__(64 * kWaves) void grouped_stream_kernel(StreamArgs 
 #pragma unroll
       for (int m = 0; m < kColTiles; ++m)
         if (m < nct)
-          *reinterpret_cast<float4*>(ep + (half * kTileTok + m * 16 + col) * kStride + cw +
+          *reinterpret_cast<float4*>(ep + (half * TT + m * 16 + col) * kStride + cw +
                                      16 * j + 4 * q) =
               make_float4(acc[j][m][0], acc[j][m][1], acc[j][m][2], acc[j][m][3]);
     __syncthreads();
@@ -311,12 +312,12 @@ __global__ __launch_bounds__(64 * kWaves) void grouped_stream_kernel(StreamArgs 
     constexpr int kGroups = kCols / 128;
     const int sub = threadIdx.x >> 4;               // 16 rows of 16 lanes
     const int li = threadIdx.x & 15;
-    for (int u = sub; u < kTileTok * kGroups; u += 16) {
+    for (int u = sub; u < TT * kGroups; u += 16) {
       const int tt = u / kGroups;
       const int cg = u - tt * kGroups;
       const int cl = cg * 128 + li * 8;             // column within the item
       const float* gp = ep + tt * kStride + cl;
-      const float* up = ep + (kTileTok + tt) * kStride + cl;
+      const float* up = ep + (TT + tt) * kStride + cl;
       const float4 g0 = *reinterpret_cast<const float4*>(gp);
       const float4 g1 = *reinterpret_cast<const float4*>(gp + 4);
       const float4 u0 = *reinterpret_cast<const float4*>(up);
@@ -403,17 +404,37 @@ static void launch_stream(const StreamArgs& A, int shape, int64_t max_tiles, hip
   const dim3 block(64 * kWaves);
   if constexpr (GLU) {
     if (shape == 2)
-      hipLaunchKernelGGL((grouped_stream_kernel<16, 4, GATHER, true>), grid, block, 0, s, A);
+      hipLaunchKernelGGL((grouped_stream_kernel<16, 4, GATHER, true, kTileTok>), grid, block, 0, s, A);
     else
-      hipLaunchKernelGGL((grouped_stream_kernel<8, 8, GATHER, true>), grid, block, 0, s, A);
+      hipLaunchKernelGGL((grouped_stream_kernel<8, 8, GATHER, true, kTileTok>), grid, block, 0, s, A);
     return;
   }
   switch (shape) {
-    case 0: hipLaunchKernelGGL((grouped_stream_kernel<16, 1, GATHER, false>), grid, block, 0, s, A); break;
-    case 1: hipLaunchKernelGGL((grouped_stream_kernel<16, 2, GATHER, false>), grid, block, 0, s, A); break;
-    case 2: hipLaunchKernelGGL((grouped_stream_kernel<16, 4, GATHER, false>), grid, block, 0, s, A); break;
-    default: hipLaunchKernelGGL((grouped_stream_kernel<8, 8, GATHER, false>), grid, block, 0, s, A); break;
+    case 0: hipLaunchKernelGGL((grouped_stream_kernel<16, 1, GATHER, false, kTileTok>), grid, block, 0, s, A); break;
+    case 1: hipLaunchKernelGGL((grouped_stream_kernel<16, 2, GATHER, false, kTileTok>), grid, block, 0, s, A); break;
+    case 2: hipLaunchKernelGGL((grouped_stream_kernel<16, 4, GATHER, false, kTileTok>), grid, block, 0, s, A); break;
+    default: hipLaunchKernelGGL((grouped_stream_kernel<8, 8, GATHER, false, kTileTok>), grid, block, 0, s, A); break;
   }
+}
+
+// Calls on 16-row tiles: up to 6 rows per expert, where nearly every tile has
+// 16 or fewer.  Half the LDS and a ring of 8 put four workgroups on a CU
+// instead of two, with as much in flight, so the last wave of items is shorter.
+// us per call, 256 experts, top-8, H 2048, I 512, 32 rows -> 16: 29 tokens
+// 101.2 -> 95.0, 64 128.4 -> 124.5, 128 142.4 -> 138.8 (uneven popularity
+// 126.1 -> 121.4), 200 146.6 -> 143.4, 300 150.3 -> 155.5 (9 rows per expert:
+// some have two tiles).
+constexpr int kSmallRowsPerExpert = 6;
+static bool use_small(int64_t P, int32_t n_experts, int32_t hidden) {
+  return hidden % 256 == 0 && P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
+}
+
+// Their launches: gate/up in the GLU form and down, both of 4 groups per wave.
+template <bool GATE_UP>
+static void launch_small(const StreamArgs& A, int64_t max_tiles, hipStream_t s) {
+  const int64_t items = max_tiles * (A.rows / 256);
+  hipLaunchKernelGGL((grouped_stream_kernel<8, 4, GATE_UP, GATE_UP, kSmallTileTok>),
+                     dim3(static_cast<unsigned>((items + 7) & ~int64_t{7})), dim3(64 * kWaves), 0, s, A);
 }
 
 // ------------------------------------------------------ SiLU * up -> e4m3
@@ -545,14 +566,22 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   int32_t* tiles = reinterpret_cast<int32_t*>(ws + L.tiles);
   int32_t* n_tiles = reinterpret_cast<int32_t*>(ws + L.n_tiles);
   const int64_t P = static_cast<int64_t>(tokens) * top_k;
-  const int64_t max_tiles = (P + kTileTok - 1) / kTileTok + n_experts;
-  // (h holds the wide tiles' records: nothing else of that path uses it)
   const bool wide = use_wide(P, n_experts, hidden);
+  const int gu_shape = pick_shape(P, n_experts, 2 * inter, kGateUpShape);
+  const bool glu = glu_shape(gu_shape, inter);
+  const bool small = !wide && glu && use_small(P, n_experts, hidden);
+  const int tile_rows = wide ? kWideTile : small ? kSmallTileTok : kTileTok;
+  // (h is free with both: it holds the records of the wide tiles, which are
+  // larger, and of the 16-row ones, which are more)
+  int32_t* const recs = wide || small ? reinterpret_cast<int32_t*>(h) : tiles;
+  // an expert of n rows has at most n tiles
+  const int64_t by_rows = (P + tile_rows - 1) / tile_rows + n_experts;
+  const int64_t max_tiles = by_rows < P ? by_rows : P;
   // the permutation and the activation rows' quantisation in one launch
   const QuantRowsJob quant{x, hidden, xq, xs, tokens};
   int rc = launch_permute(ids, ids64, P, n_experts, counts, offsets, sorted, pos, s,
-                          wide ? reinterpret_cast<int32_t*>(h) : tiles, n_tiles,
-                          wide ? kWideTile : kTileTok, &quant, wide,
+                          recs, n_tiles,
+                          tile_rows, &quant, wide,
                           reinterpret_cast<int32_t*>(y));   // y is free until the down launch
   if (rc) return rc;
   if (wide) {
@@ -562,15 +591,15 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   }
   StreamArgs gu{};
   gu.act = xq;  gu.act_s = xs;  gu.sorted = sorted;
-  gu.counts = counts;  gu.offsets = offsets;  gu.tiles = tiles;  gu.n_tiles = n_tiles;
+  gu.counts = counts;  gu.offsets = offsets;  gu.tiles = recs;  gu.n_tiles = n_tiles;
   gu.w = w13;  gu.ws = s13;  gu.out = h;  gu.w_es = es.w13;  gu.s_es = es.s13;
   gu.top_k = top_k;  gu.rows = 2 * inter;  gu.G = hidden / 128;
   gu.tiled = es.layout == MOE_LAYOUT_TILES;
   gu.aq = aq;  gu.as = as_;  gu.inter = inter;
-  const int gu_shape = pick_shape(P, n_experts, gu.rows, kGateUpShape);
-  if (glu_shape(gu_shape, inter)) {
+  if (glu) {
     // gate/up, SiLU * up and its quantisation in one launch
-    launch_stream<true, true>(gu, gu_shape, max_tiles, s);
+    if (small) launch_small<true>(gu, max_tiles, s);
+    else launch_stream<true, true>(gu, gu_shape, max_tiles, s);
     rc = check_launch("moe_fp8_moe_forward(grouped gate/up + SiLU)");
     if (rc) return rc;
   } else {
@@ -584,11 +613,12 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   }
   StreamArgs dn{};
   dn.act = aq;  dn.act_s = as_;  dn.sorted = nullptr;
-  dn.counts = counts;  dn.offsets = offsets;  dn.tiles = tiles;  dn.n_tiles = n_tiles;
+  dn.counts = counts;  dn.offsets = offsets;  dn.tiles = recs;  dn.n_tiles = n_tiles;
   dn.w = w2;  dn.ws = s2;  dn.out = y;  dn.w_es = es.w2;  dn.s_es = es.s2;
   dn.top_k = top_k;  dn.rows = hidden;  dn.G = inter / 128;
   dn.tiled = es.layout == MOE_LAYOUT_TILES;
-  launch_stream<false>(dn, pick_shape(P, n_experts, dn.rows, kDownShape), max_tiles, s);
+  if (small) launch_small<false>(dn, max_tiles, s);
+  else launch_stream<false>(dn, pick_shape(P, n_experts, dn.rows, kDownShape), max_tiles, s);
   rc = check_launch("moe_fp8_moe_forward(grouped down)");
   if (rc) return rc;
   return launch_unpermute(y, pos, weights, wbf16, tokens, top_k, hidden, residual, out, s);
