@@ -143,6 +143,14 @@ constexpr int kGateUpSplit = 2;                  // waves per tile
 constexpr int kGateUpWaves = kGateUpSplit * kGateUpTiles;
 static_assert(kGateUpTiles == 2, "a workgroup pairs one gate tile with the up tile of its columns");
 constexpr int kGateUpChunk = 8;                  // K-blocks in flight per lane
+// ... and in launches of more workgroups than fit the chip with 8 (94
+// registers: 5 per CU).  With 4 (62 registers) 8 fit: a wave waits twice, but
+// there is no second round of workgroups.  us per step of 4 resident layers
+// (top-8 of 256, H 2048, I 512: 32 workgroups per pair), 8 -> 4 in flight: 4
+// tokens (1024 workgroups) 111.2 -> 111.8, 8 (2048) 182.3 -> 177.5, 16 (4096)
+// 314 -> 303; H 1024, I 1024, whose waves have 4 K-blocks each, 16 tokens 390 -> 328.
+constexpr int kGateUpChunkMany = 4;
+constexpr int kGateUpManyFrom = 5 * 256;         // workgroups
 
 //
 // TOPK > 0 (moe_router_fp8_moe_forward): no ids are read; every wave takes
@@ -153,16 +161,22 @@ constexpr int kGateUpChunk = 8;                  // K-blocks in flight per lane
 // launch.
 // The logits' round trip and the top-k take the place of the id load ahead
 // of the weight loads, and the top-k needs no launch of its own.
-template <int SHARED, int TOPK>
+template <int SHARED, int TOPK, int CHUNK>
 __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
     const uint16_t* __restrict__ x, const void* __restrict__ ids, int ids64, int32_t top_k,
     const uint8_t* __restrict__ w13, const float* __restrict__ s13, int64_t w13_es,
     int64_t s13_es, int tiled, int32_t n_experts, int32_t hidden, int32_t inter,
     float* __restrict__ act, int32_t tokens, SharedRefs sh, const float* __restrict__ logits,
     float* __restrict__ wout) {
+  // per tile the block products (or, in a workgroup of the shared expert, its
+  // partial sums: a little more)
+  constexpr int kDpart = kGateUpTiles * (kMaxHidden / 128) * 16;
+  constexpr int kSpart = SHARED == kSharedMma ? kSharedPartFloats<1, 1, 8> : 0;
+  __shared__ __align__(16) float dpart_mem[kSpart > kDpart ? kSpart : kDpart];
+  float (*const dpart)[kMaxHidden / 128][16] =
+      reinterpret_cast<float (*)[kMaxHidden / 128][16]>(dpart_mem);
   __shared__ __align__(16) uint8_t xq[kMaxHidden];
   __shared__ float xs[kMaxHidden / 128];
-  __shared__ __align__(16) float dpart[kGateUpTiles][kMaxHidden / 128][16];
   __shared__ float spart[kGateUpTiles][kMaxHidden / 128];
   __shared__ __align__(16) float upsum[16];
   const int wave = threadIdx.x >> 6;
@@ -170,11 +184,10 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
   if (SHARED == kSharedMma && blockIdx.y >= static_cast<unsigned>(tokens * top_k)) {
     // one tile of the shared expert's gate/up: 8 columns, or the sigmoid gate
     // row, of all tokens, with the parts of K and the sums of moe_shared_gate_up
-    __shared__ float mma_part[SHARED == kSharedMma ? kSharedPartFloats<1, 1, 8> : 1];
     const int j = ((blockIdx.y - tokens * top_k) * gridDim.x + blockIdx.x) * 8;
     if (j > sh.inter) return;                    // the whole workgroup
     shared_gate_up_tile<1, 1, 8, 2, kGateUpWaves>(x, sh.wg, sh.wu, sh.wsg, tokens, hidden, sh.inter,
-                                                  sh.act, sh.sig, j, 0, mma_part);
+                                                  sh.act, sh.sig, j, 0, dpart_mem);
     return;
   }
   if (SHARED == kSharedGemv && blockIdx.y >= static_cast<unsigned>(tokens * top_k)) {
@@ -268,14 +281,14 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
   // they would add a round trip between the weights' arrival and the MFMAs)
   const float* srow =
       s13 + (valid ? e : 0) * s13_es + static_cast<int64_t>(r0 >> 7) * G;
-  float sw[kGateUpChunk];
+  float sw[CHUNK];
 #pragma unroll
-  for (int c = 0; c < kGateUpChunk; ++c) sw[c] = srow[min(gb + c, G - 1)];
+  for (int c = 0; c < CHUNK; ++c) sw[c] = srow[min(gb + c, G - 1)];
   __builtin_amdgcn_sched_barrier(0);
   PHASE_MARK(1);                       // the id is in: the weight loads go out
-  v8i a[kGateUpChunk];
+  v8i a[CHUNK];
 #pragma unroll
-  for (int c = 0; c < kGateUpChunk; ++c)
+  for (int c = 0; c < CHUNK; ++c)
     a[c] = load_op_nt(wrow + min(gb + c, G - 1) * ow.kstep, ow.half);
   __builtin_amdgcn_sched_barrier(0);   // every load above is issued before the math below
   // x[t] -> e4m3 codes + per-128 scales in LDS: 8 values per lane, 16 lanes
@@ -299,10 +312,10 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
   // leave them in LDS (lane l holds rows 4(l/16)..+3, as every lane with
   // the same l/16 does).
   v4f acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < gn; k0 += kGateUpChunk) {
+  for (int k0 = 0; k0 < gn; k0 += CHUNK) {
     if (k0 > 0) {
 #pragma unroll
-      for (int c = 0; c < kGateUpChunk; ++c)
+      for (int c = 0; c < CHUNK; ++c)
         if (k0 + c < gn) {
           a[c] = load_op_nt(wrow + (gb + k0 + c) * ow.kstep, ow.half);
           sw[c] = srow[gb + k0 + c];
@@ -310,7 +323,7 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
     }
     if (!owner) {
 #pragma unroll
-      for (int c = 0; c < kGateUpChunk; ++c) {
+      for (int c = 0; c < CHUNK; ++c) {
         const int k = k0 + c;
         if (k < gn) {
           const int g = gb + k;
@@ -327,7 +340,7 @@ __global__ __launch_bounds__(64 * kGateUpWaves) void gateup_gemv_kernel(
       }
     } else {
 #pragma unroll
-      for (int c = 0; c < kGateUpChunk; ++c) {
+      for (int c = 0; c < CHUNK; ++c) {
         const int k = k0 + c;
         if (k < gn) {
           const int g = gb + k;
@@ -948,44 +961,38 @@ static int launch_gemv(const uint16_t* x, const void* ids, int ids64, const void
   const int64_t pairs = static_cast<int64_t>(tokens) * top_k;
   const unsigned gx = static_cast<unsigned>((2 * inter) / 16);
   const bool sh_mma = sh && tokens >= kSharedMmaFrom;
+  // (a wave of at most 4 K-blocks has no use for 8 either)
+  const bool few_blocks = hidden <= 128 * kGateUpSplit * kGateUpChunkMany;
+  const bool many = few_blocks || static_cast<int64_t>(gx / kGateUpTiles) * pairs > kGateUpManyFrom;
+  constexpr int C8 = kGateUpChunk, C4 = kGateUpChunkMany;
+  auto kern = many ? gateup_gemv_kernel<kSharedNone, 0, C4> : gateup_gemv_kernel<kSharedNone, 0, C8>;
+  unsigned extra_y = 0;    // rows of workgroups of the shared expert
   if (sh_mma) {
-    // extra rows of workgroups for the shared expert's Is / 8 + 1 tiles
+    // its Is / 8 + 1 tiles; with them in the launch 4 in flight measured no better
+    // (block of 8 tokens 39.6 -> 40.9 us, of 16 74.0 -> 73.6)
     const unsigned per_y = gx / kGateUpTiles;
-    const unsigned sy = static_cast<unsigned>((sh->inter / 8 + 1 + per_y - 1) / per_y);
-    hipLaunchKernelGGL((gateup_gemv_kernel<kSharedMma, 0>), dim3(gx / kGateUpTiles, pairs + sy),
-                       dim3(64 * kGateUpWaves), 0, s, x, ids,
-                       ids64, top_k, w13, s13, es.w13, es.s13, static_cast<int>(es.layout),
-                       n_experts, hidden, inter, h, tokens, *sh, nullptr, nullptr);
+    extra_y = static_cast<unsigned>((sh->inter / 8 + 1 + per_y - 1) / per_y);
+    kern = few_blocks ? gateup_gemv_kernel<kSharedMma, 0, C4> : gateup_gemv_kernel<kSharedMma, 0, C8>;
   } else if (sh) {
-    // extra rows of workgroups for the shared expert's Is + 1 rows (the last: sigmoid gate)
+    // its Is + 1 rows (the last: sigmoid gate)
     const unsigned per_y = kSharedJPW * (gx / kGateUpTiles) * kGateUpWaves;
-    const unsigned sy = static_cast<unsigned>((sh->inter + 1 + per_y - 1) / per_y);
-    hipLaunchKernelGGL((gateup_gemv_kernel<kSharedGemv, 0>), dim3(gx / kGateUpTiles, pairs + sy),
-                       dim3(64 * kGateUpWaves), 0, s, x, ids,
-                       ids64, top_k, w13, s13, es.w13, es.s13, static_cast<int>(es.layout),
-                       n_experts, hidden, inter, h, tokens, *sh, nullptr, nullptr);
+    extra_y = static_cast<unsigned>((sh->inter + 1 + per_y - 1) / per_y);
+    kern = gateup_gemv_kernel<kSharedGemv, 0, C8>;
   } else if (rt) {
-    // one token: the ids and weights the down launch reads are the top-k's
+    // the ids and weights the down launch reads are the top-k's
     ids = rt->ids;
     ids64 = 0;
     weights = rt->weights;
     wbf16 = 0;
     if (n_experts <= 256)
-      hipLaunchKernelGGL((gateup_gemv_kernel<kSharedNone, 4>), dim3(gx / kGateUpTiles, pairs),
-                         dim3(64 * kGateUpWaves), 0, s, x, ids, 0, top_k, w13, s13, es.w13,
-                         es.s13, static_cast<int>(es.layout), n_experts, hidden, inter, h, tokens,
-                         SharedRefs{}, rt->logits, rt->weights);
+      kern = many ? gateup_gemv_kernel<kSharedNone, 4, C4> : gateup_gemv_kernel<kSharedNone, 4, C8>;
     else
-      hipLaunchKernelGGL((gateup_gemv_kernel<kSharedNone, 16>), dim3(gx / kGateUpTiles, pairs),
-                         dim3(64 * kGateUpWaves), 0, s, x, ids, 0, top_k, w13, s13, es.w13,
-                         es.s13, static_cast<int>(es.layout), n_experts, hidden, inter, h, tokens,
-                         SharedRefs{}, rt->logits, rt->weights);
-  } else {
-    hipLaunchKernelGGL((gateup_gemv_kernel<kSharedNone, 0>), dim3(gx / kGateUpTiles, pairs),
-                       dim3(64 * kGateUpWaves), 0, s, x, ids, ids64,
-                       top_k, w13, s13, es.w13, es.s13, static_cast<int>(es.layout), n_experts,
-                       hidden, inter, h, tokens, SharedRefs{}, nullptr, nullptr);
+      kern = many ? gateup_gemv_kernel<kSharedNone, 16, C4> : gateup_gemv_kernel<kSharedNone, 16, C8>;
   }
+  hipLaunchKernelGGL(kern, dim3(gx / kGateUpTiles, pairs + extra_y), dim3(64 * kGateUpWaves), 0, s,
+                     x, ids, ids64, top_k, w13, s13, es.w13, es.s13, static_cast<int>(es.layout),
+                     n_experts, hidden, inter, h, tokens, sh ? *sh : SharedRefs{},
+                     rt ? rt->logits : nullptr, rt ? rt->weights : nullptr);
   int rc = check_launch("moe_fp8_moe_forward(gate/up)");
   if (rc) return rc;
   if (sh) {
