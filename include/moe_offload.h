@@ -694,7 +694,7 @@ size_t moe_fp8_moe_block_workspace(int32_t tokens, int32_t top_k,
  *   out = bf16(residual + bf16(routed + bf16(sig * shared_down)))
  * with routed the bf16 result of moe_fp8_moe_forward_ex on the same
  * arguments and the shared terms those of moe_shared_gate_up/_down, bit for
- * bit.  On the per-pair GEMV path with at most 2 tokens (decode) the shared
+ * bit.  On the per-pair GEMV path with at most 16 tokens (decode) the shared
  * expert is carried by the two routed launches: extra workgroups of the
  * gate/up launch and one extra wave per workgroup of the down launch.  Any
  * other call runs the routed experts, then the two shared-expert kernels
