@@ -494,11 +494,13 @@ static int launch_wide(const GroupedLayout& L, char* ws, int64_t P, int32_t top_
   A.tiled = es.layout == MOE_LAYOUT_TILES;
   A.ipt = inter / 128;
   // Neighbouring tiles are mostly one expert's and share its weights in an
-  // XCD's L2; fewer than one run of four per XCD would leave XCDs idle.  Runs
-  // of 1 / 2 / 4 / 8 tiles, 256 experts, 4096 tokens: 482 / 412 / 393 / 390
-  // us; 2000 tokens of uneven popularity, runs of 4 / 8 / 16: 265 / 273 / 285;
-  // 16 experts, 100 tokens (17 tiles), 1 / 4: 40.6 / 43.0.
-  A.chunk = tiles >= 32 ? 4 : 1;
+  // XCD's L2, but few runs per XCD leave XCDs idle at the end.  Runs of 4 / 8 /
+  // 12 / 24 tiles, 256 experts, us: 4096 tokens (640 tiles) 352 / 345 / 355 /
+  // 385, of uneven popularity 360 / 354 / 358 / 391; 3000 (500) 306 / 305 / 315
+  // / 318; 2000 (370) 245.5 / 250 / 248 / 248, uneven 253 / 256 / 265 / 288.
+  // Runs of 1 / 2 / 4 at 4096 tokens with a slower permutation: 482 / 412 / 393.
+  // 16 experts, 100 tokens (17 tiles), runs of 1 / 4: 40.6 / 43.0.
+  A.chunk = tiles >= 512 ? 8 : tiles >= 32 ? 4 : 1;
   // Past the caches when the call reads about one tile of every expert and the
   // experts don't fit the 256 MB last-level cache: 1021 tokens over 256 experts
   // (805 MB) 203 -> 184 us, 300 over 64 of H 2560, I 256 (126 MB) 49 -> 56;

@@ -7,11 +7,12 @@
 // What bounds it: with 32-row tiles a call of 1021 tokens (256 experts, top-8,
 // 32 rows per expert in 1.5 tiles) read its weights 1.5 times past the
 // caches, and one of 4096 tokens four and a half times.  Here the first reads
-// them once from HBM (gate/up 5.6 TB/s of its 537 MB), the second's re-reads
-// are served by the XCDs' L2s.  Gate/up + down, us, H 2048, I 512, MI355X,
-// streamed -> wide: 1021 tokens (row order) 152 + 92 -> 107 + 65, 4096 tokens
-// 283 + 178 -> 162 + 129 (uneven popularity), where the down projection also
-// writes 268 MB of float32 rows.
+// them once from HBM (gate/up 5.6 TB/s of its 537 MB in tile order), the
+// second's re-reads are half served by the XCDs' L2s (910 MB read past them at
+// 5.5 TB/s).  us, H 2048, I 512, MI355X, streamed -> wide: 1021 tokens' call 216
+// -> 182 in tile order (gate/up 96 + down 58), 267 -> 205 in row order; 4096
+// tokens of uneven popularity, gate/up + down 283 + 178 -> 166 + 131, where down
+// also writes 268 MB of float32 rows.
 //
 // A workgroup of 8 waves takes one item: a tile and, for gate/up, one
 // 128-column group of the intermediate (each wave the gate and the up rows of
