@@ -1,0 +1,158 @@
+// Which form of a kernel serves a call: rules on sizes alone, in plain C++,
+// so that they can be evaluated on the host without a GPU.
+#pragma once
+
+#include <math.h>
+#include <stdint.h>
+
+namespace moe {
+
+// ------------------------------------------------------ grouped expert FFN
+
+constexpr int kTileTok = 32;          // permuted rows per tile (two MFMA column tiles)
+constexpr int kSmallTileTok = 16;     // the same for calls of few rows per expert
+constexpr int kWideTile = 64;         // the same for calls of many rows per expert (grouped_wide.hip)
+constexpr int kWideDownRows = 256;    // rows of w2 per row block of a wide down item
+constexpr int kMinItems = 400;        // fewest work items worth a bigger GPW
+
+// Work-item shapes, in increasing rows per item: (ring slots, groups of 16
+// rows per wave).  The last trades ring depth for rows so that the
+// accumulators of 8 groups fit beside the ring at 2 waves per SIMD.
+struct StreamShape {
+  int ring, gpw;
+};
+constexpr StreamShape kShapes[] = {{16, 1}, {16, 2}, {16, 4}, {8, 8}};
+constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
+constexpr int kGateUpShape = 2;       // (16, 4): whole 128-column groups, the GLU form
+constexpr int kDownShape = 3;         // (8, 8)
+static_assert(kGateUpShape < kNumShapes && kDownShape < kNumShapes, "shape index");
+
+// Expected tile count of P uniform picks over n_experts: each expert's
+// pair count n is Poisson(P / n_experts) and takes ceil(n / rows) tiles,
+// E[ceil(n / rows)] = sum over j >= 0 of P(n > rows * j).
+inline double expected_tiles(int64_t P, int32_t n_experts, int rows) {
+  if (P <= 0) return 0.0;
+  const double lam = static_cast<double>(P) / n_experts;
+  if (lam > 1000.0) return n_experts * (lam / rows + 0.5);
+  double tiles = 0.0, cdf = 0.0, logp = -lam;   // log P(n = 0)
+  int n = 0;
+  for (int j = 0;; ++j) {
+    const int m = rows * j;
+    for (; n <= m; ++n) {
+      cdf += exp(logp);
+      logp += log(lam) - log(static_cast<double>(n + 1));
+    }
+    const double tail = 1.0 - cdf;
+    if (m > lam && tail < 1e-9) break;
+    tiles += tail;
+  }
+  return n_experts * tiles;
+}
+
+// Shape for a projection of `rows` weight rows: the biggest up to `target`
+// that tiles the rows and still gives kMinItems work items at the expected
+// tile count (fewer items than that leave CUs idle: small calls over few
+// experts take smaller items).  Bigger items amortise each workgroup's start
+// (tile look-up, staging, first loads) and drain; the GLU form needs
+// GPW >= 4.  Measured on MI355X over 256 resident experts, top-8, H 2048,
+// I 512, T = 17 .. 1024 tokens and every pair of shapes: gate/up (16, 4)
+// with down (8, 8) was the fastest pair or within 1.5 % of it at every T.
+inline int pick_shape(int64_t P, int32_t n_experts, int32_t rows, int target) {
+  const double tiles = expected_tiles(P, n_experts, kTileTok);
+  int fallback = -1;
+  for (int i = target; i >= 0; --i) {
+    const int g = kShapes[i].gpw;
+    if (rows % (64 * g) != 0) continue;
+    fallback = i;
+    if (tiles * rows / (64.0 * g) >= kMinItems) return i;
+  }
+  return fallback < 0 ? 0 : fallback;
+}
+
+// Whether the GLU form serves a gate/up projection of this shape: items of
+// whole 128-column groups (GPW >= 4) that tile the intermediate columns.
+inline bool glu_shape(int shape, int32_t inter) {
+  const int g = kShapes[shape].gpw;
+  return g >= 4 && inter % (32 * g) == 0;
+}
+
+// Calls on 16-row tiles: up to 6 rows per expert, where nearly every tile has
+// 16 or fewer.  Half the LDS and a ring of 8 put four workgroups on a CU
+// instead of two, with as much in flight, so the last wave of items is shorter.
+// us per call, 256 experts, top-8, H 2048, I 512, 32 rows -> 16: 29 tokens
+// 101.2 -> 95.0, 64 128.4 -> 124.5, 128 142.4 -> 138.8 (uneven popularity
+// 126.1 -> 121.4), 200 146.6 -> 143.4, 300 150.3 -> 155.5 (9 rows per expert:
+// some have two tiles).
+constexpr int kSmallRowsPerExpert = 6;
+inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden) {
+  return hidden % 256 == 0 && P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
+}
+
+// Calls on the wide tiles (grouped_wide.hip): from 18 rows per expert, with w2
+// in whole row blocks.  us per call at H 2048, I 512, tile order, streamed ->
+// wide, MI355X: 256 experts top-8, 512 tokens (16 rows per expert) 159.7 ->
+// 162.0, 700 182 -> 171, 1021 216 -> 181, 2000 328 -> 258, 4096 574 -> 393;
+// 64 experts top-6, 200 tokens (19) 61.3 -> 54.5, 700 101 -> 75; 16 experts
+// top-8, 100 tokens 44.4 -> 40.6; row order, 1021 tokens 276 -> 208.
+constexpr int kWideRowsPerExpert = 18;
+inline bool use_wide(int64_t P, int32_t n_experts, int32_t hidden) {
+  return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(kWideRowsPerExpert) * n_experts;
+}
+
+// Consecutive tiles per XCD turn of the wide kernel.
+// Neighbouring tiles are mostly one expert's and share its weights in an
+// XCD's L2, but few runs per XCD leave XCDs idle at the end.  Runs of 4 / 8 /
+// 12 / 24 tiles, 256 experts, us: 4096 tokens (640 tiles) 352 / 345 / 355 /
+// 385, of uneven popularity 360 / 354 / 358 / 391; 3000 (500) 306 / 305 / 315
+// / 318; 2000 (370) 245.5 / 250 / 248 / 248, uneven 253 / 256 / 265 / 288.
+// Runs of 1 / 2 / 4 at 4096 tokens with a slower permutation: 482 / 412 / 393.
+// 16 experts, 100 tokens (17 tiles), runs of 1 / 4: 40.6 / 43.0.
+inline int wide_chunk(double tiles) { return tiles >= 512 ? 8 : tiles >= 32 ? 4 : 1; }
+
+// Whether the wide gate/up reads its weights past the caches.
+// Past the caches when the call reads about one tile of every expert and the
+// experts don't fit the 256 MB last-level cache: 1021 tokens over 256 experts
+// (805 MB) 203 -> 184 us, 300 over 64 of H 2560, I 256 (126 MB) 49 -> 56;
+// 2000 over 256 (two tiles per expert) 267 -> 272.  Row-major loads use each
+// line twice, and the down projection measured slower past the caches (1021
+// tokens 64 -> 70 us).
+inline bool wide_stream(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter, bool tiled) {
+  return tiled && P < 48LL * n_experts && 3LL * hidden * inter * n_experts > (256LL << 20);
+}
+
+// Row blocks of w2 per item of the wide down projection: two (4096 tokens, 1 /
+// 2 / 4 blocks: 137 / 127 / 133 us) while that leaves an item per CU.
+inline int wide_blocks(double tiles, int32_t hidden) {
+  const int nblk = hidden / kWideDownRows;
+  return nblk >= 2 && tiles * nblk >= 512 ? 2 : 1;
+}
+
+// How a grouped call runs.
+struct GroupedPlan {
+  int tile_rows;             // kSmallTileTok, kTileTok or kWideTile
+  int gate_up_shape, down_shape;   // kTileTok: indices of kShapes
+  bool glu;                  // gate/up with SiLU in its epilogue
+  int chunk, blocks;         // kWideTile: see above
+  bool stream;
+};
+
+inline GroupedPlan grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter,
+                                bool tiled) {
+  GroupedPlan p{};
+  if (use_wide(P, n_experts, hidden)) {
+    const double tiles = expected_tiles(P, n_experts, kWideTile);
+    p.tile_rows = kWideTile;
+    p.glu = true;
+    p.chunk = wide_chunk(tiles);
+    p.blocks = wide_blocks(tiles, hidden);
+    p.stream = wide_stream(P, n_experts, hidden, inter, tiled);
+    return p;
+  }
+  p.gate_up_shape = pick_shape(P, n_experts, 2 * inter, kGateUpShape);
+  p.glu = glu_shape(p.gate_up_shape, inter);
+  p.tile_rows = p.glu && use_small(P, n_experts, hidden) ? kSmallTileTok : kTileTok;
+  p.down_shape = pick_shape(P, n_experts, hidden, kDownShape);
+  return p;
+}
+
+}  // namespace moe

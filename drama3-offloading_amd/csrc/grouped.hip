@@ -27,11 +27,10 @@
 // scales multiply each 128-deep block result as weight_scale *
 // activation_scale, and the blocks are summed in the same order -- so every
 // (token, expert) row computed here is bit-identical to the decode GEMV's.
-#include <math.h>
-
 #include <type_traits>
 
 #include "common.hpp"
+#include "dispatch.hpp"
 #include "grouped.hpp"
 
 namespace moe {
@@ -63,15 +62,12 @@ namespace moe {
 // down 8 with a ring of 8, each stepping down only for calls too small to
 // fill the chip (pick_shape).
 
-constexpr int kTileTok = 32;          // permuted rows per tile (two MFMA column tiles)
-constexpr int kSmallTileTok = 16;     // the same for calls of few rows per expert
 constexpr int kWaves = 4;             // waves per workgroup
 constexpr int kRing = 16;             // K-block operands in flight per lane
 constexpr int kStageBlocks = 16;      // K-blocks of activations staged at a time
 constexpr int kStageRowBytes = kStageBlocks * 128;
 constexpr int kMaxGPW = 8;            // groups of 16 rows per wave
 constexpr int kMaxScaleRows = kMaxGPW / 2;   // 128-row weight-scale rows per item
-constexpr int kMinItems = 400;        // fewest work items worth a bigger GPW
 
 // LDS of one workgroup: the activation tile first (the direct loads address
 // it from offset 0), then the scales and the tile's token rows.
@@ -336,67 +332,6 @@ __global__ __launch_bounds__(64 * kWaves, TT == kSmallTileTok ? 4 : 1) void grou
   }
 }
 
-// Work-item shapes, in increasing rows per item: (ring slots, groups of 16
-// rows per wave).  The last trades ring depth for rows so that the
-// accumulators of 8 groups fit beside the ring at 2 waves per SIMD.
-struct StreamShape {
-  int ring, gpw;
-};
-constexpr StreamShape kShapes[] = {{16, 1}, {16, 2}, {16, 4}, {8, 8}};
-constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
-constexpr int kGateUpShape = 2;       // (16, 4): whole 128-column groups, the GLU form
-constexpr int kDownShape = 3;         // (8, 8)
-static_assert(kGateUpShape < kNumShapes && kDownShape < kNumShapes, "shape index");
-
-// Expected tile count of P uniform picks over n_experts: each expert's
-// pair count n is Poisson(P / n_experts) and takes ceil(n / rows) tiles,
-// E[ceil(n / rows)] = sum over j >= 0 of P(n > rows * j).
-static double expected_tiles(int64_t P, int32_t n_experts, int rows) {
-  if (P <= 0) return 0.0;
-  const double lam = static_cast<double>(P) / n_experts;
-  if (lam > 1000.0) return n_experts * (lam / rows + 0.5);
-  double tiles = 0.0, cdf = 0.0, logp = -lam;   // log P(n = 0)
-  int n = 0;
-  for (int j = 0;; ++j) {
-    const int m = rows * j;
-    for (; n <= m; ++n) {
-      cdf += exp(logp);
-      logp += log(lam) - log(static_cast<double>(n + 1));
-    }
-    const double tail = 1.0 - cdf;
-    if (m > lam && tail < 1e-9) break;
-    tiles += tail;
-  }
-  return n_experts * tiles;
-}
-
-// Shape for a projection of `rows` weight rows: the biggest up to `target`
-// that tiles the rows and still gives kMinItems work items at the expected
-// tile count (fewer items than that leave CUs idle: small calls over few
-// experts take smaller items).  Bigger items amortise each workgroup's start
-// (tile look-up, staging, first loads) and drain; the GLU form needs
-// GPW >= 4.  Measured on MI355X over 256 resident experts, top-8, H 2048,
-// I 512, T = 17 .. 1024 tokens and every pair of shapes: gate/up (16, 4)
-// with down (8, 8) was the fastest pair or within 1.5 % of it at every T.
-static int pick_shape(int64_t P, int32_t n_experts, int32_t rows, int target) {
-  const double tiles = expected_tiles(P, n_experts, kTileTok);
-  int fallback = -1;
-  for (int i = target; i >= 0; --i) {
-    const int g = kShapes[i].gpw;
-    if (rows % (64 * g) != 0) continue;
-    fallback = i;
-    if (tiles * rows / (64.0 * g) >= kMinItems) return i;
-  }
-  return fallback < 0 ? 0 : fallback;
-}
-
-// Whether the GLU form serves a gate/up projection of this shape: items of
-// whole 128-column groups (GPW >= 4) that tile the intermediate columns.
-static bool glu_shape(int shape, int32_t inter) {
-  const int g = kShapes[shape].gpw;
-  return g >= 4 && inter % (32 * g) == 0;
-}
-
 template <bool GATHER, bool GLU = false>
 static void launch_stream(const StreamArgs& A, int shape, int64_t max_tiles, hipStream_t s) {
   const int64_t items = max_tiles * (A.rows / (64 * kShapes[shape].gpw));
@@ -417,19 +352,7 @@ static void launch_stream(const StreamArgs& A, int shape, int64_t max_tiles, hip
   }
 }
 
-// Calls on 16-row tiles: up to 6 rows per expert, where nearly every tile has
-// 16 or fewer.  Half the LDS and a ring of 8 put four workgroups on a CU
-// instead of two, with as much in flight, so the last wave of items is shorter.
-// us per call, 256 experts, top-8, H 2048, I 512, 32 rows -> 16: 29 tokens
-// 101.2 -> 95.0, 64 128.4 -> 124.5, 128 142.4 -> 138.8 (uneven popularity
-// 126.1 -> 121.4), 200 146.6 -> 143.4, 300 150.3 -> 155.5 (9 rows per expert:
-// some have two tiles).
-constexpr int kSmallRowsPerExpert = 6;
-static bool use_small(int64_t P, int32_t n_experts, int32_t hidden) {
-  return hidden % 256 == 0 && P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
-}
-
-// Their launches: gate/up in the GLU form and down, both of 4 groups per wave.
+// The 16-row tiles' launches: gate/up in the GLU form and down, both of 4 groups per wave.
 template <bool GATE_UP>
 static void launch_small(const StreamArgs& A, int64_t max_tiles, hipStream_t s) {
   const int64_t items = max_tiles * (A.rows / 256);
@@ -464,23 +387,11 @@ __global__ __launch_bounds__(512) void grouped_silu_kernel(const float* __restri
 }
 
 
-// Calls on the wide tiles (grouped_wide.hip): from 18 rows per expert, with w2
-// in whole row blocks.  us per call at H 2048, I 512, tile order, streamed ->
-// wide, MI355X: 256 experts top-8, 512 tokens (16 rows per expert) 159.7 ->
-// 162.0, 700 182 -> 171, 1021 216 -> 181, 2000 328 -> 258, 4096 574 -> 393;
-// 64 experts top-6, 200 tokens (19) 61.3 -> 54.5, 700 101 -> 75; 16 experts
-// top-8, 100 tokens 44.4 -> 40.6; row order, 1021 tokens 276 -> 208.
-constexpr int kWideRowsPerExpert = 18;
-static bool use_wide(int64_t P, int32_t n_experts, int32_t hidden) {
-  return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(kWideRowsPerExpert) * n_experts;
-}
-
-static int launch_wide(const GroupedLayout& L, char* ws, int64_t P, int32_t top_k,
-                       const uint8_t* w13, const float* s13, const uint8_t* w2, const float* s2,
+static int launch_wide(const GroupedPlan& p, const GroupedLayout& L, char* ws, int64_t P,
+                       int32_t top_k, const uint8_t* w13, const float* s13, const uint8_t* w2, const float* s2,
                        const moe_expert_strides& es, int32_t n_experts, int32_t hidden,
                        int32_t inter, hipStream_t s) {
   const int64_t max_tiles = (P + kWideTile - 1) / kWideTile + n_experts;
-  const double tiles = expected_tiles(P, n_experts, kWideTile);
   WideArgs A{};
   A.act = reinterpret_cast<const uint8_t*>(ws + L.xq);
   A.act_s = reinterpret_cast<const float*>(ws + L.xs);
@@ -493,33 +404,16 @@ static int launch_wide(const GroupedLayout& L, char* ws, int64_t P, int32_t top_
   A.top_k = top_k;  A.rows = 2 * inter;  A.G = hidden / 128;  A.inter = inter;
   A.tiled = es.layout == MOE_LAYOUT_TILES;
   A.ipt = inter / 128;
-  // Neighbouring tiles are mostly one expert's and share its weights in an
-  // XCD's L2, but few runs per XCD leave XCDs idle at the end.  Runs of 4 / 8 /
-  // 12 / 24 tiles, 256 experts, us: 4096 tokens (640 tiles) 352 / 345 / 355 /
-  // 385, of uneven popularity 360 / 354 / 358 / 391; 3000 (500) 306 / 305 / 315
-  // / 318; 2000 (370) 245.5 / 250 / 248 / 248, uneven 253 / 256 / 265 / 288.
-  // Runs of 1 / 2 / 4 at 4096 tokens with a slower permutation: 482 / 412 / 393.
-  // 16 experts, 100 tokens (17 tiles), runs of 1 / 4: 40.6 / 43.0.
-  A.chunk = tiles >= 512 ? 8 : tiles >= 32 ? 4 : 1;
-  // Past the caches when the call reads about one tile of every expert and the
-  // experts don't fit the 256 MB last-level cache: 1021 tokens over 256 experts
-  // (805 MB) 203 -> 184 us, 300 over 64 of H 2560, I 256 (126 MB) 49 -> 56;
-  // 2000 over 256 (two tiles per expert) 267 -> 272.  Row-major loads use each
-  // line twice, and the down projection measured slower past the caches (1021
-  // tokens 64 -> 70 us).
-  A.stream = A.tiled && P < 48LL * n_experts &&
-             3LL * hidden * inter * n_experts > (256LL << 20);
+  A.chunk = p.chunk;
+  A.stream = p.stream;
   int rc = launch_grouped_wide(A, true, max_tiles, s);
   if (rc) return rc;
   A.act = A.aq;  A.act_s = A.as;
   A.w = w2;  A.ws = s2;  A.w_es = es.w2;  A.s_es = es.s2;
   A.out = reinterpret_cast<float*>(ws + L.y);
   A.rows = hidden;  A.G = inter / 128;
-  // two row blocks per item (4096 tokens, 1 / 2 / 4 blocks: 137 / 127 / 133
-  // us) while that leaves an item per CU
-  const int nblk = hidden / kWideDownRows;
-  A.blocks = nblk >= 2 && tiles * nblk >= 512 ? 2 : 1;
-  A.ipt = (nblk + A.blocks - 1) / A.blocks;
+  A.blocks = p.blocks;
+  A.ipt = (hidden / kWideDownRows + p.blocks - 1) / p.blocks;
   A.stream = 0;
   return launch_grouped_wide(A, false, max_tiles, s);
 }
@@ -568,11 +462,10 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   int32_t* tiles = reinterpret_cast<int32_t*>(ws + L.tiles);
   int32_t* n_tiles = reinterpret_cast<int32_t*>(ws + L.n_tiles);
   const int64_t P = static_cast<int64_t>(tokens) * top_k;
-  const bool wide = use_wide(P, n_experts, hidden);
-  const int gu_shape = pick_shape(P, n_experts, 2 * inter, kGateUpShape);
-  const bool glu = glu_shape(gu_shape, inter);
-  const bool small = !wide && glu && use_small(P, n_experts, hidden);
-  const int tile_rows = wide ? kWideTile : small ? kSmallTileTok : kTileTok;
+  const GroupedPlan plan =
+      grouped_plan(P, n_experts, hidden, inter, es.layout == MOE_LAYOUT_TILES);
+  const int tile_rows = plan.tile_rows;
+  const bool wide = tile_rows == kWideTile, small = tile_rows == kSmallTileTok;
   // (h is free with both: it holds the records of the wide tiles, which are
   // larger, and of the 16-row ones, which are more)
   int32_t* const recs = wide || small ? reinterpret_cast<int32_t*>(h) : tiles;
@@ -587,7 +480,7 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
                           reinterpret_cast<int32_t*>(y));   // y is free until the down launch
   if (rc) return rc;
   if (wide) {
-    rc = launch_wide(L, ws, P, top_k, w13, s13, w2, s2, es, n_experts, hidden, inter, s);
+    rc = launch_wide(plan, L, ws, P, top_k, w13, s13, w2, s2, es, n_experts, hidden, inter, s);
     if (rc) return rc;
     return launch_unpermute(y, pos, weights, wbf16, tokens, top_k, hidden, residual, out, s);
   }
@@ -598,14 +491,14 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   gu.top_k = top_k;  gu.rows = 2 * inter;  gu.G = hidden / 128;
   gu.tiled = es.layout == MOE_LAYOUT_TILES;
   gu.aq = aq;  gu.as = as_;  gu.inter = inter;
-  if (glu) {
+  if (plan.glu) {
     // gate/up, SiLU * up and its quantisation in one launch
     if (small) launch_small<true>(gu, max_tiles, s);
-    else launch_stream<true, true>(gu, gu_shape, max_tiles, s);
+    else launch_stream<true, true>(gu, plan.gate_up_shape, max_tiles, s);
     rc = check_launch("moe_fp8_moe_forward(grouped gate/up + SiLU)");
     if (rc) return rc;
   } else {
-    launch_stream<true>(gu, gu_shape, max_tiles, s);
+    launch_stream<true>(gu, plan.gate_up_shape, max_tiles, s);
     rc = check_launch("moe_fp8_moe_forward(grouped gate/up)");
     if (rc) return rc;
     hipLaunchKernelGGL(grouped_silu_kernel, dim3(static_cast<unsigned>((P + 7) / 8)), dim3(512), 0,
@@ -620,7 +513,7 @@ int launch_grouped(const uint16_t* x, const void* ids, int ids64, const void* we
   dn.top_k = top_k;  dn.rows = hidden;  dn.G = inter / 128;
   dn.tiled = es.layout == MOE_LAYOUT_TILES;
   if (small) launch_small<false>(dn, max_tiles, s);
-  else launch_stream<false>(dn, pick_shape(P, n_experts, dn.rows, kDownShape), max_tiles, s);
+  else launch_stream<false>(dn, plan.down_shape, max_tiles, s);
   rc = check_launch("moe_fp8_moe_forward(grouped down)");
   if (rc) return rc;
   return launch_unpermute(y, pos, weights, wbf16, tokens, top_k, hidden, residual, out, s);

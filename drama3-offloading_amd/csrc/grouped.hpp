@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "dispatch.hpp"
 
 namespace moe {
 
@@ -64,8 +65,6 @@ int launch_unpermute(const float* y, const int32_t* pair_pos, const void* weight
 // kWideTile rows (the tiles the permute launch listed).
 // A tile's record is (expert, first permuted row, rows of its expert from
 // there on, unused).
-constexpr int kWideTile = 64;
-constexpr int kWideDownRows = 256;   // rows of w2 per row block of a down item
 struct WideArgs {
   const uint8_t* act;      // activation rows, e4m3, G*128 bytes each
   const float* act_s;      // their per-128 scales, G per row
