@@ -95,7 +95,28 @@ inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden) {
 // 64 experts top-6, 200 tokens (19) 61.3 -> 54.5, 700 101 -> 75; 16 experts
 // top-8, 100 tokens 44.4 -> 40.6; row order, 1021 tokens 276 -> 208.
 constexpr int kWideRowsPerExpert = 18;
-inline bool use_wide(int64_t P, int32_t n_experts, int32_t hidden) {
+// ... and with enough of them to fill the chip: a call of a few tiles takes as
+// long as one item, a chain of hidden / 128 K-blocks that the streamed kernel
+// cuts into more and smaller items (pick_shape).  So at least kWideMinItems
+// gate/up items (tiles x 128-column groups), growing as the square root of
+// hidden, and below kWideFewTiles tiles at least half of each filled.  us,
+// streamed / wide, weights not in the caches, tile order: H 2048, I 512, 1
+// expert of 64 rows (6 items) 27.5 / 31.3, 2 of 128 (20) 28.9 / 32.6, 8 of 48
+// (33) 0.91 x the wide time, 8 of 64 (48) 1.09 x; H 4096, I 384, 1 of 64 (5)
+// 34.0 / 42.7, 8 of 64 (36) 48.7 / 52.4, 16 of 64 (72) 61.1 / 60.9; H 8192, I
+// 2048, 1 of 64 (24) 61.4 / 93.6, 4 of 24 (64) 0.84 x, 4 of 64 (96) 131.8 /
+// 103.0.  In row order, H 1024, I 1024, 8 of 24 rows (64 items of 8 tiles) 0.88
+// x, 8 of 32 1.02 x, 16 of 24 1.23 x; H 2048, I 512, 12 of 24 (48) 0.93 x, 12 of
+// 32 1.16 x.
+constexpr int kWideMinItems = 38;
+constexpr int kWideFewTiles = 14, kWideFewTilesRows = 32;
+inline bool enough_wide_items(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter,
+                              double tiles) {
+  const double items = tiles * (inter / 128);
+  if (tiles < kWideFewTiles && P < static_cast<int64_t>(kWideFewTilesRows) * n_experts) return false;
+  return items >= kWideMinItems && items * items >= 0.75 * hidden;
+}
+inline bool enough_wide_rows(int64_t P, int32_t n_experts, int32_t hidden) {
   return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(kWideRowsPerExpert) * n_experts;
 }
 
@@ -139,8 +160,9 @@ struct GroupedPlan {
 inline GroupedPlan grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter,
                                 bool tiled) {
   GroupedPlan p{};
-  if (use_wide(P, n_experts, hidden)) {
-    const double tiles = expected_tiles(P, n_experts, kWideTile);
+  const double tiles = enough_wide_rows(P, n_experts, hidden)
+                           ? expected_tiles(P, n_experts, kWideTile) : 0.0;
+  if (enough_wide_items(P, n_experts, hidden, inter, tiles)) {
     p.tile_rows = kWideTile;
     p.glu = true;
     p.chunk = wide_chunk(tiles);

@@ -241,3 +241,44 @@ def test_wide_tiles_equal_gemv(lib, dev, T, E, K, H, I, tiled):
     assert torch.equal(*outs)
     bad = torch.isnan(outs[0].view(torch.bfloat16)).any(1).nonzero().view(-1).tolist()
     assert bad == ([3, T - 1] if T > 64 and E > 1 else [])
+
+
+# rows per expert around whole tiles and column tiles of 16, one expert without
+# any; repeated to the number of experts
+_SEGMENTS = (64, 65, 128, 129, 63, 1, 17, 0, 16, 33, 48, 127)
+
+
+@pytest.mark.parametrize("E,used,H,I", [
+    (60, 60, 256, 128),          # one K-block of the down projection, two of gate/up
+    (24, 24, 768, 384),          # a row block to spare, windows that end inside K
+    (12, 12, 2048, 512), (12, 12, 8192, 2048),   # the largest expert
+    (240, 180, 1024, 512),       # weights past the caches, in tile order
+])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_wide_tiles_segment_edges(lib, dev, E, used, H, I, tiled):
+    """Wide tiles of segments that fill, miss and overrun them by a row,
+    bit-identical to the per-pair GEMV."""
+    from hostpool import RecordLayout
+    import hipfetch
+    counts = [_SEGMENTS[e % len(_SEGMENTS)] if e < used else 0 for e in range(E)]
+    g = torch.Generator().manual_seed(E + H)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ids = ids[torch.randperm(len(ids), generator=g)].view(-1, 1).to(dev)
+    T = len(ids)
+    devt = _device_experts(E, E, H, I, dev)
+    if tiled:
+        lay = RecordLayout(H, I)
+        devt = lay.views(torch.cat([lay.pack(*(t[e:e + 1] for t in devt)) for e in range(E)]))
+    x = torch.randn((T, H), generator=g).to(torch.bfloat16).to(dev)
+    w = torch.rand((T, 1), generator=g).to(dev)
+    say(f"wide tiles, segment edges: T={T} E={E} H={H} I={I} tiled={tiled}")
+    outs = []
+    for mode in (1, 2):
+        out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
+        ws = torch.empty(lib.fp8_moe_workspace(T, 1, E, H, I), dtype=torch.uint8, device=dev)
+        lib.fp8_moe_forward(x, ids, w, devt[0].view(torch.float8_e4m3fn), devt[1],
+                            devt[2].view(torch.float8_e4m3fn), devt[3], out, ws, mode=mode,
+                            layout=hipfetch.LAYOUT_TILES if tiled else hipfetch.LAYOUT_ROWS)
+        torch.cuda.synchronize()
+        outs.append(out.view(torch.int16))
+    assert torch.equal(*outs)
