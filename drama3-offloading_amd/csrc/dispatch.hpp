@@ -88,13 +88,29 @@ inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden) {
   return hidden % 256 == 0 && P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
 }
 
-// Calls on the wide tiles (grouped_wide.hip): from 18 rows per expert, with w2
-// in whole row blocks.  us per call at H 2048, I 512, tile order, streamed ->
+// Calls on the wide tiles (grouped_wide.hip): by rows per expert, with w2 in
+// whole row blocks.  us per call at H 2048, I 512, tile order, streamed ->
 // wide, MI355X: 256 experts top-8, 512 tokens (16 rows per expert) 159.7 ->
-// 162.0, 700 182 -> 171, 1021 216 -> 181, 2000 328 -> 258, 4096 574 -> 393;
-// 64 experts top-6, 200 tokens (19) 61.3 -> 54.5, 700 101 -> 75; 16 experts
-// top-8, 100 tokens 44.4 -> 40.6; row order, 1021 tokens 276 -> 208.
-constexpr int kWideRowsPerExpert = 18;
+// 162.0, 700 182 -> 171, 1021 216 -> 181, 2000 328 -> 258, 4096 574 -> 393; 64
+// experts top-6, 700 tokens 101 -> 75; row order, 1021 tokens 276 -> 208.
+// Streamed over wide at 18 and 20 rows, mean (range) over 64 to 256 experts of
+// six shapes, evenly routed and by Zipf(1.1) popularity: tile order 0.99 (0.89
+// .. 1.19) and 1.01 (0.91 .. 1.18), row order 1.05 (0.88 .. 1.34) and 1.09 (0.88
+// .. 1.36).  Tile order, weights past the last-level cache, gate/up items of
+// fewer than 16 K-blocks (their start and epilogue show) against streamed
+// down items of a long K: H 1024, I 1024, 256 experts, 20 rows 0.94 / 0.94, 24
+// 0.97 / 0.97, 28 0.98 / 0.99, 40 1.27 / 1.05.
+constexpr int kWideRowsTiled = 20, kWideRowsRows = 18, kWideRowsShortItems = 28;
+inline bool experts_past_cache(int32_t n_experts, int32_t hidden, int32_t inter) {
+  return 3LL * hidden * inter * n_experts > (256LL << 20);
+}
+inline bool enough_wide_rows(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter,
+                             bool tiled) {
+  const bool short_items =
+      hidden < 2048 && inter > 512 && experts_past_cache(n_experts, hidden, inter);
+  const int rows = !tiled ? kWideRowsRows : short_items ? kWideRowsShortItems : kWideRowsTiled;
+  return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(rows) * n_experts;
+}
 // ... and with enough of them to fill the chip: a call of a few tiles takes as
 // long as one item, a chain of hidden / 128 K-blocks that the streamed kernel
 // cuts into more and smaller items (pick_shape).  So at least kWideMinItems
@@ -116,10 +132,6 @@ inline bool enough_wide_items(int64_t P, int32_t n_experts, int32_t hidden, int3
   if (tiles < kWideFewTiles && P < static_cast<int64_t>(kWideFewTilesRows) * n_experts) return false;
   return items >= kWideMinItems && items * items >= 0.75 * hidden;
 }
-inline bool enough_wide_rows(int64_t P, int32_t n_experts, int32_t hidden) {
-  return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(kWideRowsPerExpert) * n_experts;
-}
-
 // Consecutive tiles per XCD turn of the wide kernel.
 // Neighbouring tiles are mostly one expert's and share its weights in an
 // XCD's L2, but few runs per XCD leave XCDs idle at the end.  Runs of 4 / 8 /
@@ -138,7 +150,7 @@ inline int wide_chunk(double tiles) { return tiles >= 512 ? 8 : tiles >= 32 ? 4 
 // line twice, and the down projection measured slower past the caches (1021
 // tokens 64 -> 70 us).
 inline bool wide_stream(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter, bool tiled) {
-  return tiled && P < 48LL * n_experts && 3LL * hidden * inter * n_experts > (256LL << 20);
+  return tiled && P < 48LL * n_experts && experts_past_cache(n_experts, hidden, inter);
 }
 
 // Row blocks of w2 per item of the wide down projection: two (4096 tokens, 1 /
@@ -160,7 +172,7 @@ struct GroupedPlan {
 inline GroupedPlan grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter,
                                 bool tiled) {
   GroupedPlan p{};
-  const double tiles = enough_wide_rows(P, n_experts, hidden)
+  const double tiles = enough_wide_rows(P, n_experts, hidden, inter, tiled)
                            ? expected_tiles(P, n_experts, kWideTile) : 0.0;
   if (enough_wide_items(P, n_experts, hidden, inter, tiles)) {
     p.tile_rows = kWideTile;

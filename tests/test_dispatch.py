@@ -77,3 +77,29 @@ def test_few_experts_take_the_streamed_tiles(rules, case):
 def test_enough_items_take_the_wide_tiles(rules, case):
     H, I, E, rows = case
     assert grouped_plan(rules, rows * E, E, 1, H, I).tile_rows == 64
+
+
+# (hidden, inter, experts, rows of each, tile order): timed slower on the wide
+# tiles, evenly routed or by popularity, and faster
+FEW_ROWS_STREAMED = [
+    (2048, 512, 64, 18, True), (4096, 384, 192, 18, True), (1024, 512, 192, 18, True),
+    (1024, 1024, 256, 18, True), (1024, 1024, 256, 24, True), (1024, 1024, 192, 24, True),
+    (2048, 512, 256, 16, False),
+]
+ENOUGH_ROWS_WIDE = [
+    (2048, 512, 256, 20, True), (2048, 512, 64, 22, True), (2048, 1024, 64, 22, True),
+    (1024, 1024, 256, 28, True), (1024, 1024, 64, 24, True), (2048, 512, 256, 18, False),
+    (2560, 256, 64, 18, False), (1024, 1024, 256, 20, False), (2048, 512, 256, 31, False),
+]
+
+
+@pytest.mark.parametrize("case", FEW_ROWS_STREAMED)
+def test_few_rows_take_the_streamed_tiles(rules, case):
+    H, I, E, rows, tiled = case
+    assert grouped_plan(rules, rows * E, E, 1, H, I, tiled).tile_rows == 32
+
+
+@pytest.mark.parametrize("case", ENOUGH_ROWS_WIDE)
+def test_enough_rows_take_the_wide_tiles(rules, case):
+    H, I, E, rows, tiled = case
+    assert grouped_plan(rules, rows * E, E, 1, H, I, tiled).tile_rows == 64
