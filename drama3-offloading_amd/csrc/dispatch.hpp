@@ -76,16 +76,26 @@ inline bool glu_shape(int shape, int32_t inter) {
   return g >= 4 && inter % (32 * g) == 0;
 }
 
-// Calls on 16-row tiles: up to 6 rows per expert, where nearly every tile has
-// 16 or fewer.  Half the LDS and a ring of 8 put four workgroups on a CU
-// instead of two, with as much in flight, so the last wave of items is shorter.
-// us per call, 256 experts, top-8, H 2048, I 512, 32 rows -> 16: 29 tokens
-// 101.2 -> 95.0, 64 128.4 -> 124.5, 128 142.4 -> 138.8 (uneven popularity
-// 126.1 -> 121.4), 200 146.6 -> 143.4, 300 150.3 -> 155.5 (9 rows per expert:
-// some have two tiles).
-constexpr int kSmallRowsPerExpert = 6;
-inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden) {
-  return hidden % 256 == 0 && P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
+// Calls on 16-row tiles: up to 5 rows per expert, of experts up to 2560 x 512.
+// Half the LDS and a ring of 8 put four workgroups on a CU instead of two, with
+// as much in flight, so the last wave of items is shorter.  An expert picked by
+// more than 16 tokens has its weights read once per 16 rows, past the caches:
+// rare with even picks, but with uneven ones the busiest experts have most of
+// the tokens, and what they re-read grows with the experts' size and the rows.
+// (Reading crowded experts through the caches instead: 102 spilled registers
+// for a second copy of the loop, and slower for even picks as the only one.)
+// us, 32 rows -> 16, MI355X, top-8 of 256, H 2048, I 512, even picks: 32 tokens
+// 103.5 -> 98.1, 64 131.5 -> 127.0, 128 149.7 -> 142.2, 190 157.1 -> 148.5.  Time of
+// 32 rows over that of 16, picks by gate logits plus log popularity (the most
+// uneven, 54 experts of 256 for 128 tokens): 48 tokens 1.13, 68 0.99, 78 0.96, 88
+// 0.98, 98 1.03, 128 1.10, 158 1.07, 178 0.96, 188 0.92; H 2560, I 512 the same to
+// 0.03 (188: 0.89); H 3072, I 512: 80 0.92; H 4096, I 384: even 96 0.96, uneven 112
+// 0.83; H 2048, I 1024: uneven 80 0.91, 160 0.98.
+constexpr int kSmallRowsPerExpert = 5;
+constexpr int32_t kSmallExpert = 2560 * 512;
+inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter) {
+  return hidden % 256 == 0 && hidden * inter <= kSmallExpert &&
+         P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
 }
 
 // Calls on the wide tiles (grouped_wide.hip): by rows per expert, with w2 in
@@ -184,7 +194,7 @@ inline GroupedPlan grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, in
   }
   p.gate_up_shape = pick_shape(P, n_experts, 2 * inter, kGateUpShape);
   p.glu = glu_shape(p.gate_up_shape, inter);
-  p.tile_rows = p.glu && use_small(P, n_experts, hidden) ? kSmallTileTok : kTileTok;
+  p.tile_rows = p.glu && use_small(P, n_experts, hidden, inter) ? kSmallTileTok : kTileTok;
   p.down_shape = pick_shape(P, n_experts, hidden, kDownShape);
   return p;
 }

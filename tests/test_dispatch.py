@@ -103,3 +103,19 @@ def test_few_rows_take_the_streamed_tiles(rules, case):
 def test_enough_rows_take_the_wide_tiles(rules, case):
     H, I, E, rows, tiled = case
     assert grouped_plan(rules, rows * E, E, 1, H, I, tiled).tile_rows == 64
+
+
+# (hidden, inter, experts, tokens) of top-8 calls timed on MI355X: on 16-row
+# tiles slower when a few experts take most picks (the first also when none
+# do), and faster
+FEW_ROWS_NOT_SMALL = [(4096, 384, 256, 96), (3072, 512, 256, 80), (2048, 1024, 256, 80),
+                      (8192, 512, 128, 80), (2048, 512, 256, 188), (2048, 512, 128, 92)]
+FEW_ROWS_SMALL = [(2048, 512, 256, 29), (2048, 512, 256, 128), (2048, 512, 256, 160),
+                  (1024, 1024, 256, 128), (2560, 512, 256, 58), (2560, 256, 256, 96)]
+
+
+def test_sixteen_row_tiles(rules):
+    rows = {c: grouped_plan(rules, c[3], c[2], 8, *c[:2]).tile_rows
+            for c in FEW_ROWS_NOT_SMALL + FEW_ROWS_SMALL}
+    assert [rows[c] for c in FEW_ROWS_NOT_SMALL] == [32] * len(FEW_ROWS_NOT_SMALL)
+    assert [rows[c] for c in FEW_ROWS_SMALL] == [16] * len(FEW_ROWS_SMALL)
