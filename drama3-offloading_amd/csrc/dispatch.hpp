@@ -199,4 +199,26 @@ inline GroupedPlan grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, in
   return p;
 }
 
+// ------------------------------------------------------------------ router
+
+// Whether the float64 matrix-core logits run four (2 x 2) tiles of 16 experts
+// x 16 tokens per workgroup instead of one.  A tile takes 6/7 of the time
+// there, but padded experts are whole tiles and a call lasts as long as its
+// busiest CU, so: two workgroups per CU or more, and the busiest CU's tiles,
+// padding included, at most 7/6 of its share of single ones.  us per
+// moe_router_topk call, H 2048, MI355X, one tile / four: 256 experts, 2048
+// tokens 54.8 / 47.5, 3000 77.1 / 66.7, 4096 100.5 / 85.9; 1500 (376
+// workgroups) 47.0 / 48.6, 2300 (576) 60.3 / 66.3; 144 experts, 4096 (640:
+// 2.5 per CU) 61.3 / 66.3, 8192 112.7 / 104.3; 16 experts (half of every
+// workgroup padding), 16384 38.0 / 53.0; 48 (a quarter), 8192 46.2 / 50.4;
+// 80, 8192 69.8 / 69.5; 112, 8192 90.8 / 86.6.  2 x 4 tiles: 256 experts,
+// 4096 tokens 85; 4 x 4 162.  The float64 MFMAs alone are 55 us there.
+inline bool router_four_tiles(int32_t tokens, int32_t n_experts) {
+  constexpr int64_t kCus = 256;
+  const int64_t four = static_cast<int64_t>((n_experts + 31) / 32) * ((tokens + 31) / 32);
+  const int64_t one = static_cast<int64_t>((n_experts + 15) / 16) * ((tokens + 15) / 16);
+  const int64_t busiest = 4 * ((four + kCus - 1) / kCus);
+  return four >= 2 * kCus && busiest * 6 * kCus <= one * 7;
+}
+
 }  // namespace moe

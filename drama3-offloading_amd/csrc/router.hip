@@ -22,6 +22,7 @@
 // XCD has its own L2, and a device-scope fence inside a kernel costs more
 // than a launch.
 #include "common.hpp"
+#include "dispatch.hpp"
 #include "fetch.hpp"
 #include "resolve.hpp"
 #include "route.hpp"
@@ -198,12 +199,6 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 // operands to float64 per MFMA; several tiles share the conversions (one
 // operand per MFMA at 2 x 2).
 constexpr int kLogitMmaFrom = 64;       // tokens from which this form runs
-// Workgroups of 2 x 2 tiles from which they are used: two per CU.  MI355X, 256
-// experts, H 2048, one tile -> four (moe.route, with the top-k): 4096 tokens
-// (1024 workgroups) 111 -> 86 us; 1500 (376: one CU in two has two) 47.0 ->
-// 48.6; 2 x 4 tiles 85 and 49, 4 x 4 162.  The float64 MFMAs alone are 55 us at
-// 4096 tokens.
-constexpr int kLogitMmaBigFrom = 512;
 
 __device__ __forceinline__ double bf16_elem(u32x4 v, int m) {
   const uint32_t w = m < 2 ? v.x : m < 4 ? v.y : m < 6 ? v.z : v.w;
@@ -415,9 +410,9 @@ int launch_router_logits(const void* x, const void* w, const float* bias, int32_
   const dim3 grid((n_experts + kLogitWaves - 1) / kLogitWaves,
                   (tokens + kTokBlock - 1) / kTokBlock);
   if (tokens >= kLogitMmaFrom && hidden % 32 == 0) {
-    const unsigned gx = (n_experts + 31) / 32, gy = (tokens + 31) / 32;
-    if (static_cast<int64_t>(gx) * gy >= kLogitMmaBigFrom)
-      hipLaunchKernelGGL((router_logits_mma_kernel<2, 2, 4, 4>), dim3(gx, gy), dim3(64 * 4), 0, s,
+    if (router_four_tiles(tokens, n_experts))
+      hipLaunchKernelGGL((router_logits_mma_kernel<2, 2, 4, 4>),
+                         dim3((n_experts + 31) / 32, (tokens + 31) / 32), dim3(64 * 4), 0, s,
                          static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), bias,
                          tokens, hidden, n_experts, bf16_logits, logits);
     else

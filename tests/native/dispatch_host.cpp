@@ -15,3 +15,7 @@ extern "C" void grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, int32
   const int v[7] = {p.tile_rows, p.gate_up_shape, p.down_shape, p.glu, p.chunk, p.blocks, p.stream};
   for (int i = 0; i < 7; ++i) out[i] = v[i];
 }
+
+extern "C" int router_four_tiles(int32_t tokens, int32_t n_experts) {
+  return moe::router_four_tiles(tokens, n_experts);
+}

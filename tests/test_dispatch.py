@@ -119,3 +119,14 @@ def test_sixteen_row_tiles(rules):
             for c in FEW_ROWS_NOT_SMALL + FEW_ROWS_SMALL}
     assert [rows[c] for c in FEW_ROWS_NOT_SMALL] == [32] * len(FEW_ROWS_NOT_SMALL)
     assert [rows[c] for c in FEW_ROWS_SMALL] == [16] * len(FEW_ROWS_SMALL)
+
+
+def test_router_tiles(rules):
+    """(experts, tokens) timed on MI355X, H 2048: slower with four tiles per
+    workgroup (padded experts, CUs left idle at the end), and faster."""
+    one = [(8, 16384), (16, 16384), (16, 65535), (33, 8192), (48, 8192), (48, 20000), (144, 4096),
+           (256, 1500), (256, 64)]
+    four = [(256, 2048), (256, 3000), (256, 4096), (128, 4096), (64, 8192), (32, 16384),
+            (17, 65535), (96, 8192), (144, 8192), (512, 1500)]
+    assert [rules.router_four_tiles(T, E) for E, T in one] == [0] * len(one)
+    assert [rules.router_four_tiles(T, E) for E, T in four] == [1] * len(four)

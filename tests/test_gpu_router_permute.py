@@ -176,7 +176,8 @@ def test_route_resolve_equals_router_then_resolve(lib, dev, logit_dtype):
 
 
 @pytest.mark.parametrize("E,H,T", [(320, 1056, 100), (256, 2048, 64), (40, 96, 65),
-                                   (330, 160, 1500), (40, 96, 8200), (256, 2048, 2050)])
+                                   (330, 160, 1500), (40, 96, 8200), (256, 2048, 2050),
+                                   (232, 160, 4087), (256, 2048, 2048), (17, 96, 16384)])
 def test_router_logits_matrix_cores_equal_vector_kernel(lib, dev, E, H, T):
     """From 64 tokens the logits run on the float64 matrix cores: the same
     logits, ids and weights as the vector kernel (the same call cut into
