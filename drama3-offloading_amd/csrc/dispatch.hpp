@@ -221,4 +221,33 @@ inline bool router_four_tiles(int32_t tokens, int32_t n_experts) {
   return four >= 2 * kCus && busiest * 6 * kCus <= one * 7;
 }
 
+// ----------------------------------------------------------- shared expert
+
+// Fewest tokens of the matrix-core form.  Both kernels, H 2048, Is 512, a
+// graph over 40 layers' weights on MI355X, GEMV form -> matrix cores (us per
+// call, gate/up + down): 3 tokens 5.2 + 6.6 -> 4.8 + 3.8, 4 tokens 5.6 + 7.6
+// -> 5.0 + 3.8, 16 tokens 15.2 + 23.4 -> 5.9 + 3.9, 512 tokens 389 + 640 ->
+// 22.6 + 16.3.  One or two tokens stay on the GEMV form, whose sums the
+// decode launches that carry the shared expert reproduce.
+constexpr int kSharedMmaFrom = 3;
+
+// Whether the block call carries the shared expert in the GEMV launches (up to
+// 16 tokens, one tile of its matrix-core form); otherwise the routed call is
+// followed by the two shared-expert kernels, with the same bits.  Carried, it
+// saves two launches, but the down launch has a workgroup per token, so w_down is
+// read once per token instead of once: up to 24 Mi of tokens x hidden x inter.
+// us per block, MI355X, 64 experts top-8, carried / followed: H 2048, Is 512
+// (routed I 512), 3 tokens 22.0 / 27.1, 16 71.9 / 76.7; Is 1024, 8 47.1 / 48.1, 16
+// 80.2 / 77.4; Is 2048, 4 34.4 / 36.2, 6 47.0 / 44.6, 16 101.8 / 82.0; Is 8192, 8 136.6 /
+// 76.1; H 4096, Is 512 (384), 11 81.4 / 83.2, 16 112.1 / 110.9; Is 1024, 4 43.8 / 44.3,
+// 6 59.2 / 57.2; H 8192, Is 512 (1024), 4 142.9 / 151.0, 8 267.9 / 269.8, 16 520.5 / 511.7;
+// Is 8192, 3 253.0 / 179.8.  One or two tokens are carried on the vector units.
+constexpr int32_t kCarrySharedMaxTokens = 16;
+constexpr int64_t kCarrySharedMaxWork = 24 << 20;
+inline bool block_carries_shared(int32_t tokens, int32_t hidden, int32_t shared_inter) {
+  if (tokens < kSharedMmaFrom) return true;
+  return tokens <= kCarrySharedMaxTokens &&
+         static_cast<int64_t>(tokens) * hidden * shared_inter < kCarrySharedMaxWork;
+}
+
 }  // namespace moe

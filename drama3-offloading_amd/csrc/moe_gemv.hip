@@ -1067,10 +1067,6 @@ using namespace moe;
 // re-read of shared experts costs less than the grouped path's four
 // launches up to 16 tokens.
 constexpr int32_t kGemvMaxTokens = 16;
-// The block call carries the shared expert in the GEMV launches up to this
-// many tokens (one tile of its matrix-core form); beyond, the routed call is
-// followed by the two shared-expert kernels.
-constexpr int32_t kCarrySharedMaxTokens = 16;
 
 static bool use_grouped(int32_t tokens, int32_t hidden, int32_t mode) {
   if (mode == 1 || mode == 3) return false;
@@ -1349,7 +1345,8 @@ extern "C" int moe_fp8_moe_block_forward(const void* x, const void* ids, int32_t
                       static_cast<const uint16_t*>(shared->w_up),
                       static_cast<const uint16_t*>(shared->w_down),
                       static_cast<const uint16_t*>(shared->w_sgate), Is, act, sig};
-  if (mode != 3 && !use_grouped(tokens, hidden, mode) && tokens <= kCarrySharedMaxTokens) {
+  if (mode != 3 && !use_grouped(tokens, hidden, mode) &&
+      block_carries_shared(tokens, hidden, Is)) {
     // decode: the shared expert rides in the two GEMV launches, residual last
     const int rc = forward_impl(x, ids, ids_dtype, weights, w_dtype, tokens, top_k, w13, s13,
                                 w2, s2, n_experts, hidden, inter, strides, residual, out,

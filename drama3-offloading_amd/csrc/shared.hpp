@@ -4,6 +4,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "dispatch.hpp"
 
 namespace moe {
 
@@ -234,14 +235,6 @@ __device__ __forceinline__ void shared_down_chain(const uint16_t* const (&rows)[
     for (int u = 0; u < U; ++u) ch[u].fold(acc, c0 + u < nchunk);
   }
 }
-
-// Fewest tokens of the matrix-core form.  Both kernels, H 2048, Is 512, a
-// graph over 40 layers' weights on MI355X, GEMV form -> matrix cores (us per
-// call, gate/up + down): 3 tokens 5.2 + 6.6 -> 4.8 + 3.8, 4 tokens 5.6 + 7.6
-// -> 5.0 + 3.8, 16 tokens 15.2 + 23.4 -> 5.9 + 3.9, 512 tokens 389 + 640 ->
-// 22.6 + 16.3.  One or two tokens stay on the GEMV form, whose sums the
-// decode launches that carry the shared expert reproduce.
-constexpr int kSharedMmaFrom = 3;
 
 // Launchers of the standalone shared-expert kernels (shared.hip).
 int launch_shared_gate_up(const uint16_t* x, const uint16_t* wg, const uint16_t* wu,

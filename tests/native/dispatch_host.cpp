@@ -19,3 +19,7 @@ extern "C" void grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, int32
 extern "C" int router_four_tiles(int32_t tokens, int32_t n_experts) {
   return moe::router_four_tiles(tokens, n_experts);
 }
+
+extern "C" int block_carries_shared(int32_t tokens, int32_t hidden, int32_t shared_inter) {
+  return moe::block_carries_shared(tokens, hidden, shared_inter);
+}

@@ -130,3 +130,15 @@ def test_router_tiles(rules):
             (17, 65535), (96, 8192), (144, 8192), (512, 1500)]
     assert [rules.router_four_tiles(T, E) for E, T in one] == [0] * len(one)
     assert [rules.router_four_tiles(T, E) for E, T in four] == [1] * len(four)
+
+
+def test_block_carries_the_shared_expert(rules):
+    """(hidden, shared inter, tokens) timed on MI355X: carried by the decode
+    launches where that is faster than the two shared-expert kernels after
+    them, and always for one or two tokens."""
+    carried = [(2048, 512, 3), (2048, 512, 16), (2048, 1024, 8), (2048, 2048, 4), (4096, 512, 11),
+               (4096, 384, 12), (4096, 1024, 4), (8192, 128, 16), (8192, 8192, 2), (128, 128, 16)]
+    after = [(2048, 1024, 16), (2048, 2048, 6), (2048, 4096, 4), (2048, 8192, 3), (4096, 512, 16),
+             (4096, 1024, 6), (4096, 2048, 3), (8192, 2048, 3), (8192, 8192, 3), (2048, 512, 17)]
+    assert [rules.block_carries_shared(T, H, Is) for H, Is, T in carried] == [1] * len(carried)
+    assert [rules.block_carries_shared(T, H, Is) for H, Is, T in after] == [0] * len(after)

@@ -103,7 +103,22 @@ def test_block_forward_equals_composition(lib, dev, T, K, mode):
     """moe_fp8_moe_block_forward (the shared expert carried by the decode
     launches when T <= 16) against the composition of the three
     separate calls, bit for bit, with and without the residual."""
-    E, H, I, Is = 24, 2048, 512, 512
+    _block_against_composition(lib, dev, T, K, mode, 24, 2048, 512, 512)
+
+
+@pytest.mark.parametrize("H,I,Is", [
+    (1024, 512, 384),            # 4 K-blocks in flight; the down chain's last chunks partial
+    (640, 256, 640),             # more shared columns than routed; K-blocks of no whole chunk
+    (4096, 384, 384), (128, 128, 1280),
+    (2048, 512, 4096),           # not carried from 3 tokens
+])
+@pytest.mark.parametrize("T", [2, 3, 9, 16])
+def test_block_forward_shapes(lib, dev, T, H, I, Is):
+    """The same for other shapes, the shared expert's inner size not the routed one."""
+    _block_against_composition(lib, dev, T, 6, 0, 12, H, I, Is)
+
+
+def _block_against_composition(lib, dev, T, K, mode, E, H, I, Is):
     w13, s13, w2, s2 = _routed_experts(T * 31 + K, E, H, I, dev)
     g = torch.Generator(device="cpu").manual_seed(T + K)
     bf = lambda *s, std=1.0: (torch.randn(s, generator=g) * std).to(torch.bfloat16).to(dev)
@@ -112,7 +127,7 @@ def test_block_forward_equals_composition(lib, dev, T, K, mode):
     ids = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)]).to(torch.int32).to(dev)
     w = torch.softmax(torch.randn((T, K), generator=g), -1).to(dev)
     ws = torch.empty(lib.fp8_moe_block_workspace(T, K, E, H, I, Is), dtype=torch.uint8, device=dev)
-    say(f"block forward: T={T} K={K} mode={mode}")
+    say(f"block forward: T={T} K={K} mode={mode} H={H} I={I} Is={Is}")
     for r in (None, res):
         got = torch.empty_like(x)
         lib.fp8_moe_block_forward(x, ids, w, w13, s13, w2, s2, sh, got, ws, mode=mode, residual=r)
