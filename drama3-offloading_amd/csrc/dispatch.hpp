@@ -250,4 +250,26 @@ inline bool block_carries_shared(int32_t tokens, int32_t hidden, int32_t shared_
          static_cast<int64_t>(tokens) * hidden * shared_inter < kCarrySharedMaxWork;
 }
 
+// ------------------------------------------------- decode GEMV's gate/up
+
+// Whether a gate/up wave, with wave_blocks K-blocks of weights, keeps 4 of them
+// in flight instead of 8.  8 take 94 registers (5 workgroups per CU), 4 take 62
+// (8 per CU), so a launch of more than 5 workgroups per CU has no second round
+// of them, but a wave of 7 or 8 blocks waits twice instead of once.  Waves of 4
+// blocks or fewer have no use for 8, shorter ones than 7 little (the loads past
+// the last block repeat it), and longer ones wait several times anyway; a wave
+// that makes the router's top-k first (topk) is late with its loads, so there
+// more workgroups count for more.  us, MI355X, top-8 of 256, 8 -> 4 in flight:
+// H 2048, I 512, ids given, 8 tokens (2048 workgroups) 37.2 -> 38.1, 12 52.0 ->
+// 53.4, 16 66.9 -> 68.1; top-k inside 44.1 -> 43.1, 60.4 -> 59.6, 76.9 -> 74.6, 4 tokens
+// (1024) 26.9 -> 27.1; ids given, H 1280, I 512, 12 tokens 37.0 -> 34.4, H 1536
+// 40.8 -> 39.2, H 1792 45.9 -> 45.7; H 2560, I 256, 12 tokens (1536) 39.8 -> 39.0; H
+// 8192, I 512 (of 64), 16 245.6 -> 242.2; H 1024, I 1024, top-k inside, 16 tokens,
+// per 4 layers 390 -> 328.  With the shared expert's tiles in the launch 4 were no
+// better (block of 8 tokens 39.6 -> 40.9, of 16 74.0 -> 73.6).
+inline bool gateup_four_in_flight(int wave_blocks, int64_t workgroups, bool topk) {
+  if (wave_blocks <= 4) return true;
+  return workgroups > 5 * 256 && (topk || wave_blocks < 7 || wave_blocks > 8);
+}
+
 }  // namespace moe

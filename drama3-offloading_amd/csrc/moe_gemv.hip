@@ -27,6 +27,7 @@
 // lets kernel 1's waves take the top-k of the logits themselves instead of
 // reading ids (gateup_gemv_kernel's TOPK).
 #include "common.hpp"
+#include "dispatch.hpp"
 #include "gemv.hpp"
 #include "grouped.hpp"
 #include "route.hpp"
@@ -143,14 +144,7 @@ constexpr int kGateUpSplit = 2;                  // waves per tile
 constexpr int kGateUpWaves = kGateUpSplit * kGateUpTiles;
 static_assert(kGateUpTiles == 2, "a workgroup pairs one gate tile with the up tile of its columns");
 constexpr int kGateUpChunk = 8;                  // K-blocks in flight per lane
-// ... and in launches of more workgroups than fit the chip with 8 (94
-// registers: 5 per CU).  With 4 (62 registers) 8 fit: a wave waits twice, but
-// there is no second round of workgroups.  us per step of 4 resident layers
-// (top-8 of 256, H 2048, I 512: 32 workgroups per pair), 8 -> 4 in flight: 4
-// tokens (1024 workgroups) 111.2 -> 111.8, 8 (2048) 182.3 -> 177.5, 16 (4096)
-// 314 -> 303; H 1024, I 1024, whose waves have 4 K-blocks each, 16 tokens 390 -> 328.
-constexpr int kGateUpChunkMany = 4;
-constexpr int kGateUpManyFrom = 5 * 256;         // workgroups
+constexpr int kGateUpChunkMany = 4;              // ... where gateup_four_in_flight
 
 //
 // TOPK > 0 (moe_router_fp8_moe_forward): no ids are read; every wave takes
@@ -961,18 +955,18 @@ static int launch_gemv(const uint16_t* x, const void* ids, int ids64, const void
   const int64_t pairs = static_cast<int64_t>(tokens) * top_k;
   const unsigned gx = static_cast<unsigned>((2 * inter) / 16);
   const bool sh_mma = sh && tokens >= kSharedMmaFrom;
-  // (a wave of at most 4 K-blocks has no use for 8 either)
-  const bool few_blocks = hidden <= 128 * kGateUpSplit * kGateUpChunkMany;
-  const bool many = few_blocks || static_cast<int64_t>(gx / kGateUpTiles) * pairs > kGateUpManyFrom;
+  const int32_t wave_blocks = (hidden / 128 + kGateUpSplit - 1) / kGateUpSplit;
+  const bool many = gateup_four_in_flight(wave_blocks, static_cast<int64_t>(gx / kGateUpTiles) * pairs,
+                                          rt != nullptr);
   constexpr int C8 = kGateUpChunk, C4 = kGateUpChunkMany;
   auto kern = many ? gateup_gemv_kernel<kSharedNone, 0, C4> : gateup_gemv_kernel<kSharedNone, 0, C8>;
   unsigned extra_y = 0;    // rows of workgroups of the shared expert
   if (sh_mma) {
-    // its Is / 8 + 1 tiles; with them in the launch 4 in flight measured no better
-    // (block of 8 tokens 39.6 -> 40.9 us, of 16 74.0 -> 73.6)
+    // its Is / 8 + 1 tiles
     const unsigned per_y = gx / kGateUpTiles;
     extra_y = static_cast<unsigned>((sh->inter / 8 + 1 + per_y - 1) / per_y);
-    kern = few_blocks ? gateup_gemv_kernel<kSharedMma, 0, C4> : gateup_gemv_kernel<kSharedMma, 0, C8>;
+    kern = gateup_four_in_flight(wave_blocks, 0, false) ? gateup_gemv_kernel<kSharedMma, 0, C4>
+                                                        : gateup_gemv_kernel<kSharedMma, 0, C8>;
   } else if (sh) {
     // its Is + 1 rows (the last: sigmoid gate)
     const unsigned per_y = kSharedJPW * (gx / kGateUpTiles) * kGateUpWaves;

@@ -23,3 +23,7 @@ extern "C" int router_four_tiles(int32_t tokens, int32_t n_experts) {
 extern "C" int block_carries_shared(int32_t tokens, int32_t hidden, int32_t shared_inter) {
   return moe::block_carries_shared(tokens, hidden, shared_inter);
 }
+
+extern "C" int gateup_four_in_flight(int wave_blocks, int64_t workgroups, int topk) {
+  return moe::gateup_four_in_flight(wave_blocks, workgroups, topk != 0);
+}

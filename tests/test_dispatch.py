@@ -24,6 +24,7 @@ def build_rules(tmp_path_factory):
     lib.expected_tiles.argtypes = [ctypes.c_int64, ctypes.c_int32, ctypes.c_int]
     lib.expected_tiles.restype = ctypes.c_double
     lib.grouped_plan.argtypes = [ctypes.c_int64] + [ctypes.c_int32] * 4 + [ctypes.c_void_p]
+    lib.gateup_four_in_flight.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int]
     return lib
 
 
@@ -142,3 +143,19 @@ def test_block_carries_the_shared_expert(rules):
              (4096, 1024, 6), (4096, 2048, 3), (8192, 2048, 3), (8192, 8192, 3), (2048, 512, 17)]
     assert [rules.block_carries_shared(T, H, Is) for H, Is, T in carried] == [1] * len(carried)
     assert [rules.block_carries_shared(T, H, Is) for H, Is, T in after] == [0] * len(after)
+
+
+def test_gate_up_loads_in_flight(rules):
+    """(hidden, inter, tokens, top-k inside) of top-8 calls timed on MI355X:
+    faster with 8 K-blocks of weights in flight, and with 4."""
+    eight = [(2048, 512, 8, 0), (2048, 512, 16, 0), (1920, 512, 12, 0), (2048, 512, 4, 1),
+             (2560, 256, 4, 0), (8192, 512, 2, 1)]
+    four = [(2048, 512, 8, 1), (2048, 512, 16, 1), (2560, 256, 12, 0), (4096, 384, 8, 0),
+            (8192, 512, 16, 0), (1024, 512, 1, 0), (1024, 1024, 16, 1), (1280, 512, 12, 0),
+            (1536, 512, 8, 0)]
+
+    def rule(H, I, T, topk):
+        return rules.gateup_four_in_flight((H // 128 + 1) // 2, I // 16 * T * 8, topk)
+
+    assert [rule(*c) for c in eight] == [0] * len(eight)
+    assert [rule(*c) for c in four] == [1] * len(four)
