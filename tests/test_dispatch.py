@@ -9,6 +9,8 @@ from pathlib import Path
 import pytest
 from scipy import stats
 
+from test_gpu_grouped import WIDE_PLANS
+
 ROOT = Path(__file__).resolve().parent
 Plan = namedtuple("Plan", "tile_rows gate_up_shape down_shape glu chunk blocks stream")
 
@@ -104,6 +106,13 @@ def test_few_rows_take_the_streamed_tiles(rules, case):
 def test_enough_rows_take_the_wide_tiles(rules, case):
     H, I, E, rows, tiled = case
     assert grouped_plan(rules, rows * E, E, 1, H, I, tiled).tile_rows == 64
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+def test_wide_plans_of_the_gpu_cases(rules, tiled):
+    for (T, E, K, H, I), want in WIDE_PLANS.items():
+        p = grouped_plan(rules, T, E, K, H, I, tiled)
+        assert (p.tile_rows, p.chunk, p.blocks) == (64, *want), (T, E, K, H, I)
 
 
 # (hidden, inter, experts, tokens) of top-8 calls timed on MI355X: on 16-row

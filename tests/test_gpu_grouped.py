@@ -282,3 +282,44 @@ def test_wide_tiles_segment_edges(lib, dev, E, used, H, I, tiled):
         torch.cuda.synchronize()
         outs.append(out.view(torch.int16))
     assert torch.equal(*outs)
+
+
+# (tokens, experts, top_k, hidden, inter) -> (chunk, row blocks per down item)
+# of the wide plan (tests/test_dispatch.py holds the plans to it)
+WIDE_PLANS = {
+    (800, 64, 8, 1024, 1024): (4, 2),    # two K windows of down kept over two row blocks
+    (800, 64, 8, 1024, 1152): (4, 2),    # three, staged again for the second block
+    (900, 64, 8, 1280, 640): (4, 2),     # an odd number of row blocks: the last item has one
+    (900, 64, 8, 1280, 1152): (4, 2),
+    (1560, 520, 8, 256, 128): (8, 1),   # runs of 8 tiles
+    (1560, 520, 8, 512, 256): (8, 2),
+}
+
+
+@pytest.mark.parametrize("case", list(WIDE_PLANS), ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("tiled", [False, True])
+def test_wide_down_row_blocks(lib, dev, case, tiled):
+    """Wide down items of two row blocks and runs of 8 tiles, bit-identical to
+    the per-pair GEMV."""
+    from hostpool import RecordLayout
+    import hipfetch
+    T, E, K, H, I = case
+    devt = _device_experts(T + H, E, H, I, dev)
+    if tiled:
+        lay = RecordLayout(H, I)
+        devt = lay.views(torch.cat([lay.pack(*(t[e:e + 1] for t in devt)) for e in range(E)]))
+    g = torch.Generator().manual_seed(T + I)
+    ids = torch.rand((T, E), generator=g).topk(K, 1).indices.to(torch.int32).to(dev)
+    w = torch.rand((T, K), generator=g).to(dev)
+    x = torch.randn((T, H), generator=g).to(torch.bfloat16).to(dev)
+    say(f"wide down: T={T} E={E} K={K} H={H} I={I} tiled={tiled}")
+    outs = []
+    for mode in (1, 2):
+        out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
+        ws = torch.empty(lib.fp8_moe_workspace(T, K, E, H, I), dtype=torch.uint8, device=dev)
+        lib.fp8_moe_forward(x, ids, w, devt[0].view(torch.float8_e4m3fn), devt[1],
+                            devt[2].view(torch.float8_e4m3fn), devt[3], out, ws, mode=mode,
+                            layout=hipfetch.LAYOUT_TILES if tiled else hipfetch.LAYOUT_ROWS)
+        torch.cuda.synchronize()
+        outs.append(out.view(torch.int16))
+    assert torch.equal(*outs)

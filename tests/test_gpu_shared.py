@@ -74,11 +74,12 @@ def test_shared_matrix_core_shapes(lib, dev, T, H, Is):
     test_shared_expert_matches_oracle, and nothing written past the tokens.
 
     act = silu(g) * u of sums that cancel has no bound in ulps of itself: a
-    product of bf16 values is exact in float32 and a wave's chain is at most
-    H / 8 + 8 float32 additions, so each sum may be off by (H / 8 + 8) *
-    2^-24 of the sum of its products' magnitudes before it is rounded, and
-    act by that through silu (slope at most 1.1) and the product; the ulps
-    are counted beyond it.  The sigmoid and the down half are judged as they
+    product of bf16 values is exact in float32, the longest of the eight
+    waves' chains has n = 64 ceil(ceil(H / 64) / 8) of them (K goes out in
+    whole 64-wide chunks) and 7 partial sums follow, so each sum may be off
+    by (n + 7) * 2^-24 of the sum of its products' magnitudes before it is
+    rounded, and act by that through silu (slope at most 1.1) and the
+    product; the ulps are counted beyond it.  The sigmoid and the down half are judged as they
     stand (sigmoid's argument enters absolutely, the residual is of order 1)."""
     p = _weights(T + H + Is, T, H, Is, dev)
     act = torch.full((T + 1, Is), 7.0, dtype=torch.bfloat16, device=dev)
@@ -98,7 +99,8 @@ def test_shared_matrix_core_shapes(lib, dev, T, H, Is):
     q = {k: _np(v) for k, v in p.items()}
     want_a, want_s = shared.gate_up(q["x"], q["wg"], q["wu"], q["wsg"])
     got_a, got_s = _np(act[:T]), sig[:T].cpu().numpy()
-    d = [(H / 8 + 8) * 2.0 ** -24 * (np.abs(q["x"]) @ np.abs(q[w]).T) for w in ("wg", "wu")]
+    chain = 64 * -(-(-(-H // 64)) // 8)
+    d = [(chain + 7) * 2.0 ** -24 * (np.abs(q["x"]) @ np.abs(q[w]).T) for w in ("wg", "wu")]
     g, u = (q["x"].astype(np.float64) @ q[w].T.astype(np.float64) for w in ("wg", "wu"))
     slack = 1.1 * d[0] * (np.abs(u) + d[1]) + np.abs(g) * d[1]
     off = got_a.astype(np.float64) - want_a
@@ -111,19 +113,23 @@ def test_shared_matrix_core_shapes(lib, dev, T, H, Is):
         assert same >= 0.99 and ulps <= 2.0, (name, same, ulps)
 
 
-def test_shared_down_in_place(lib, dev):
-    """out may alias routed (the decode step writes the block sum over it)."""
-    T, H, Is = 2, 512, 256
+@pytest.mark.parametrize("T", [2, 16, 129])
+def test_shared_down_in_place(lib, dev, T):
+    """out may alias routed (the decode step writes the block sum over it) or
+    residual: the vector form, and the matrix-core form of one and of two
+    token tiles."""
+    H, Is = 512, 256
     p = _weights(5, T, H, Is, dev)
     act = torch.empty((T, Is), dtype=torch.bfloat16, device=dev)
     sig = torch.empty(T, dtype=torch.float32, device=dev)
     lib.shared_gate_up(p["x"], p["wg"], p["wu"], p["wsg"], act, sig)
     sep = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
     lib.shared_down(act, sig, p["wd"], sep, routed=p["routed"], residual=p["res"])
-    r = p["routed"].clone()
-    lib.shared_down(act, sig, p["wd"], r, routed=r, residual=p["res"])
-    torch.cuda.synchronize()
-    assert torch.equal(r, sep)
+    for name in ("routed", "res"):
+        q = dict(p, **{name: p[name].clone()})
+        lib.shared_down(act, sig, p["wd"], q[name], routed=q["routed"], residual=q["res"])
+        torch.cuda.synchronize()
+        assert torch.equal(q[name], sep), name
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
