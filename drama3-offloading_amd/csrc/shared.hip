@@ -20,7 +20,8 @@
 // lane's 16-byte slices in row order, then the 64 lane sums (wave_sum_f32).
 //
 // From kSharedMmaFrom tokens both products run on the bf16 matrix cores
-// instead (the *_mma kernels below).
+// instead (the *_mma kernels below), whose sums have another order, the same
+// in every tile form: gate/up eight parts of K, down one chain.
 #include "shared.hpp"
 
 namespace moe {

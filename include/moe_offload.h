@@ -570,7 +570,14 @@ int moe_gather_plan(const int32_t* uniq, const int32_t* n_unique,
  *   act [tokens, inter] bf16 = bf16(silu(bf16(x w_gate^T))) * bf16(x w_up^T)
  *   sig [tokens] f32 = bf16(sigmoid(bf16(x w_sgate^T)))  (bf16 values)
  * Each product rounds to bf16 as the model's bf16 modules do.  hidden and
- * inter positive multiples of 128; x and weights 16-byte aligned. */
+ * inter positive multiples of 128; x and weights 16-byte aligned.
+ * The float32 sums run in one order in calls of one or two tokens (vector
+ * units) and in another from three on (matrix cores), there and in
+ * moe_shared_down.  The outputs' error against 64 bits is the same (3.549e-3
+ * for act at hidden 2048, that of the bf16 roundings), but a token computed
+ * alone and in a batch may differ in the last bf16 place.  Among calls of
+ * three tokens or more, and of one or two, a token's bits do not depend on the
+ * others. */
 int moe_shared_gate_up(const void* x, const void* w_gate, const void* w_up,
                        const void* w_sgate, int32_t tokens, int32_t hidden,
                        int32_t inter, void* act, float* sig, void* stream);
@@ -694,8 +701,11 @@ size_t moe_fp8_moe_block_workspace(int32_t tokens, int32_t top_k,
  *   out = bf16(residual + bf16(routed + bf16(sig * shared_down)))
  * with routed the bf16 result of moe_fp8_moe_forward_ex on the same
  * arguments and the shared terms those of moe_shared_gate_up/_down, bit for
- * bit.  On the per-pair GEMV path with at most 16 tokens (decode) the shared
- * expert is carried by the two routed launches: extra workgroups of the
+ * bit (so a token's shared terms may differ in the last bf16 place between
+ * calls of one or two tokens and larger ones; the routed ones do not).  On
+ * the per-pair GEMV path with at most 16 tokens (decode) the shared expert,
+ * unless it is large (from 3 tokens, tokens x hidden x shared inter of 24 Mi
+ * or more), is carried by the two routed launches: extra workgroups of the
  * gate/up launch and one extra wave per workgroup of the down launch.  Any
  * other call runs the routed experts, then the two shared-expert kernels
  * on its output.  No counterpart in the reference: upstream's MoE block

@@ -113,6 +113,32 @@ def test_shared_matrix_core_shapes(lib, dev, T, H, Is):
         assert same >= 0.99 and ulps <= 2.0, (name, same, ulps)
 
 
+@pytest.mark.parametrize("H,Is", [(2048, 512), (640, 384)])
+def test_shared_bits_do_not_depend_on_the_batch(lib, dev, H, Is):
+    """A token's act, sig and out have the same bits in every call of three
+    tokens or more (every tile form of the matrix cores) and in every call of
+    one or two."""
+    T = 150
+    p = _weights(H + Is, T, H, Is, dev)
+
+    def run(t0, t1):
+        act = torch.empty((t1 - t0, Is), dtype=torch.bfloat16, device=dev)
+        sig = torch.empty(t1 - t0, dtype=torch.float32, device=dev)
+        out = torch.empty((t1 - t0, H), dtype=torch.bfloat16, device=dev)
+        lib.shared_gate_up(p["x"][t0:t1], p["wg"], p["wu"], p["wsg"], act, sig)
+        lib.shared_down(act, sig, p["wd"], out, routed=p["routed"][t0:t1],
+                        residual=p["res"][t0:t1])
+        torch.cuda.synchronize()
+        return act, sig, out
+
+    whole = run(0, T)
+    for t0, n in ((0, 3), (7, 16), (20, 33), (50, 70), (1, 129)):
+        for a, b in zip(run(t0, t0 + n), whole):
+            assert torch.equal(a, b[t0:t0 + n]), (t0, n)
+    for a, b in zip(run(4, 5), run(4, 6)):
+        assert torch.equal(a, b[:1])
+
+
 @pytest.mark.parametrize("T", [2, 16, 129])
 def test_shared_down_in_place(lib, dev, T):
     """out may alias routed (the decode step writes the block sum over it) or
