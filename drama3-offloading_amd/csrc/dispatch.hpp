@@ -253,9 +253,10 @@ inline bool block_carries_shared(int32_t tokens, int32_t hidden, int32_t shared_
 // ------------------------------------------------- decode GEMV's gate/up
 
 // Whether a gate/up wave, with wave_blocks K-blocks of weights, keeps 4 of them
-// in flight instead of 8.  8 take 94 registers (5 workgroups per CU), 4 take 62
-// (8 per CU), so a launch of more than 5 workgroups per CU has no second round
-// of them, but a wave of 7 or 8 blocks waits twice instead of once.  Waves of 4
+// in flight instead of 8.  8 take 104 registers (4 workgroups per CU), 4 take 72
+// (7 per CU), so a launch of more workgroups than that has fewer rounds of them
+// (the line is at 5 per CU: with top-k inside, 1280 took 31.8 -> 31.2 at H 2048, I
+// 512, 1024 26.9 -> 27.1), but a wave of 7 or 8 blocks waits twice instead of once.  Waves of 4
 // blocks or fewer have no use for 8, shorter ones than 7 little (the loads past
 // the last block repeat it), and longer ones wait several times anyway; a wave
 // that makes the router's top-k first (topk) is late with its loads, so there

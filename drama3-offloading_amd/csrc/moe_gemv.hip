@@ -1054,12 +1054,13 @@ using namespace moe;
 
 // Calls of at most this many tokens take the per-pair GEMV kernels by default;
 // larger ones the grouped kernels, which read each expert's weights once.
-// Measured on MI355X (top-8 of 256 uniform, H 2048, I 512, tile-ordered
-// records rotating over 2048 of them, graph of back-to-back calls): GEMV
-// 9.7 / 20.9 / 37.3 / 68.7 us against grouped 47.4 / 56.1 / 54.8 / 68.7 us
-// at 1 / 4 / 8 / 16 tokens, and 82.4 against 77.5 us at 20: the GEMV's
-// re-read of shared experts costs less than the grouped path's four
-// launches up to 16 tokens.
+// us, MI355X, H 2048, I 512, tile order, weights not in the caches, GEMV /
+// grouped: top-8 of 256, even picks, 4 tokens 21.7 / 41.1, 8 37.1 / 51.8, 12 52.1 /
+// 67.1, 16 67.6 / 70.3, 18 75.5 / 74.3, 20 82.2 / 77.9; top-6 of 64, 16 50.4 / 56.5, 18
+// 56.3 / 47.6.  The GEMV reads an expert once per pick, so the line is lower where
+// picks are uneven: by Zipf(1.1) popularity, 12 49.0 / 50.3, 16 62.1 / 53.3; by gate
+// logits plus log popularity, 8 33.7 / 35.7, 10 39.2 / 36.9, 16 56.6 / 37.4.  Nothing
+// known before the launch tells them apart.
 constexpr int32_t kGemvMaxTokens = 16;
 
 static bool use_grouped(int32_t tokens, int32_t hidden, int32_t mode) {
