@@ -106,18 +106,24 @@ inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inte
 // Streamed over wide at 18 and 20 rows, mean (range) over 64 to 256 experts of
 // six shapes, evenly routed and by Zipf(1.1) popularity: tile order 0.99 (0.89
 // .. 1.19) and 1.01 (0.91 .. 1.18), row order 1.05 (0.88 .. 1.34) and 1.09 (0.88
-// .. 1.36).  Tile order, weights past the last-level cache, gate/up items of
-// fewer than 16 K-blocks (their start and epilogue show) against streamed
-// down items of a long K: H 1024, I 1024, 256 experts, 20 rows 0.94 / 0.94, 24
-// 0.97 / 0.97, 28 0.98 / 0.99, 40 1.27 / 1.05.
-constexpr int kWideRowsTiled = 20, kWideRowsRows = 18, kWideRowsShortItems = 28;
-inline bool experts_past_cache(int32_t n_experts, int32_t hidden, int32_t inter) {
-  return 3LL * hidden * inter * n_experts > (256LL << 20);
+// .. 1.36).  Tile order, gate/up items of fewer than 16 K-blocks (their start
+// and epilogue show) of experts well past the last-level cache, where the
+// streamed form runs at HBM's rate while most experts have one of its tiles:
+// H 1024, I 1024, 256 experts (805 MB), 20 rows 0.94 / 0.94, 28 0.98 / 0.99, 32 1.10 /
+// 1.00, 40 1.27 / 1.05; H 1024, I 512, 512 experts (805 MB), 22 0.98 / 0.93, 32 1.07 /
+// 0.97, but of 256 experts (403 MB) 22 1.10 / 0.95; fewer than 8 K-blocks: H 256, I
+// 512, 1000 experts (393 MB), 22 0.78 / 0.83, 32 0.88 / 0.87, 64 1.26 / 1.21; H 768, I
+// 384, 512 (453 MB), 22 0.94 / 0.90, 32 1.02 / 0.92.
+constexpr int kWideRowsTiled = 20, kWideRowsRows = 18, kWideRowsShortItems = 32;
+constexpr int64_t kLastLevelCache = 256 << 20;   // bytes
+inline int64_t expert_set_bytes(int32_t n_experts, int32_t hidden, int32_t inter) {
+  return 3LL * hidden * inter * n_experts;
 }
 inline bool enough_wide_rows(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter,
                              bool tiled) {
-  const bool short_items =
-      hidden < 2048 && inter > 512 && experts_past_cache(n_experts, hidden, inter);
+  const int64_t bytes = expert_set_bytes(n_experts, hidden, inter);
+  const bool short_items = (hidden < 1024 && bytes > kLastLevelCache) ||
+                           (hidden < 2048 && bytes > 2 * kLastLevelCache);
   const int rows = !tiled ? kWideRowsRows : short_items ? kWideRowsShortItems : kWideRowsTiled;
   return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(rows) * n_experts;
 }
@@ -160,7 +166,8 @@ inline int wide_chunk(double tiles) { return tiles >= 512 ? 8 : tiles >= 32 ? 4 
 // line twice, and the down projection measured slower past the caches (1021
 // tokens 64 -> 70 us).
 inline bool wide_stream(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter, bool tiled) {
-  return tiled && P < 48LL * n_experts && experts_past_cache(n_experts, hidden, inter);
+  return tiled && P < 48LL * n_experts &&
+         expert_set_bytes(n_experts, hidden, inter) > kLastLevelCache;
 }
 
 // Row blocks of w2 per item of the wide down projection: two (4096 tokens, 1 /
