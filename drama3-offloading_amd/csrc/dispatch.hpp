@@ -90,11 +90,15 @@ inline bool glu_shape(int shape, int32_t inter) {
 // uneven, 54 experts of 256 for 128 tokens): 48 tokens 1.13, 68 0.99, 78 0.96, 88
 // 0.98, 98 1.03, 128 1.10, 158 1.07, 178 0.96, 188 0.92; H 2560, I 512 the same to
 // 0.03 (188: 0.89); H 3072, I 512: 80 0.92; H 4096, I 384: even 96 0.96, uneven 112
-// 0.83; H 2048, I 1024: uneven 80 0.91, 160 0.98.
+// 0.83; H 2048, I 1024: uneven 80 0.91, 160 0.98.  A down item is 256 rows, half
+// the streamed one: at I 128, one K-block, too short for what it costs to start
+// (top-8 of 1000, even, 2 rows per expert: H 512 1.08, 1024 1.00, 2048 0.96, 4096
+// 0.91; uneven, 4 rows: 1.01, 0.96, 0.88, 0.79).
 constexpr int kSmallRowsPerExpert = 5;
 constexpr int32_t kSmallExpert = 2560 * 512;
 inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter) {
   return hidden % 256 == 0 && hidden * inter <= kSmallExpert &&
+         (inter > 128 || hidden <= 1024) &&
          P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
 }
 
