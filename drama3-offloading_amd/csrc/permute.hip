@@ -90,9 +90,9 @@ __device__ __forceinline__ void put_tile(int32_t* tiles, int32_t n, int32_t e, i
   }
 }
 
-// WIDE: the records of grouped_wide.hip, which need each expert's first row and
-// count; kept out of the other form, where holding them over the scan took it
-// from 60 to 78 registers and 104 to 108 us (32768 pairs of 4096 experts).
+// WIDE: the records of grouped_wide.hip, with each expert's first row and count.
+// Those are read back from the cursors: holding them over the scan took the
+// kernel from 60 to 78 registers and 104 to 108 us (32768 pairs of 4096 experts).
 template <bool WIDE>
 __global__ __launch_bounds__(kPlaceThreads) void permute_kernel(
     const void* __restrict__ ids, int ids64, int64_t P, int32_t n_experts,
@@ -165,7 +165,6 @@ __global__ __launch_bounds__(kPlaceThreads) void permute_kernel(
     // for every tile_tokens rows of every expert's segment, in expert order
     int32_t nt[kPlacePer];
     int32_t tsum = 0;
-    if constexpr (WIDE) base -= sum;   // back to the thread's first expert
 #pragma unroll
     for (int j = 0; j < kPlacePer; ++j) {
       nt[j] = (mine[j] + tile_tokens - 1) / tile_tokens;
@@ -176,9 +175,13 @@ __global__ __launch_bounds__(kPlaceThreads) void permute_kernel(
 #pragma unroll
     for (int j = 0; j < kPlacePer; ++j) {
       const int x = tid * kPlacePer + j;
+      int32_t first = 0, rows = 0;
+      if (WIDE && x < n_experts) {
+        first = cursor[x];
+        rows = (x + 1 < n_experts ? cursor[x + 1] : total) - first;
+      }
       for (int32_t i = 0; i < nt[j]; ++i)
-        put_tile(tiles, tbase + i, x, WIDE ? base : 0, WIDE ? mine[j] : 0, i * tile_tokens, WIDE);
-      if constexpr (WIDE) base += mine[j];
+        put_tile(tiles, tbase + i, x, first, rows, i * tile_tokens, WIDE);
       tbase += nt[j];
     }
     if (tid == 0) *n_tiles = ttotal;
