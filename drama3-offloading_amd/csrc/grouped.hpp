@@ -50,8 +50,8 @@ __device__ __forceinline__ void quant_row(const QuantRowsJob& q, int64_t t, int 
 // wide_tiles: the records of grouped_wide.hip in `tiles` instead (int4).
 // hist (nullable): scratch of ceil(P / 4096) * n_experts counts, with which a
 // call of several placement passes runs them side by side.
-// quant (nullable): activation rows quantised by extra workgroups of the
-// same launch, two tokens each, beside the one that permutes.
+// quant (nullable): activation rows quantised by extra workgroups of the same
+// launches, beside those that permute.
 int launch_permute(const void* ids, int ids64, int64_t P, int32_t n_experts, int32_t* counts,
                    int32_t* offsets, int32_t* sorted_pairs, int32_t* pair_pos, hipStream_t s,
                    int32_t* tiles = nullptr, int32_t* n_tiles = nullptr, int32_t tile_tokens = 16,

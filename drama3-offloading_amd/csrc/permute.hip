@@ -255,23 +255,32 @@ constexpr int kFastExperts = 1024;                      // one thread per expert
 // SPLIT: one workgroup per pass, for calls of several passes that have the
 // passes' counts already (hist [passes][E], permute_count_kernel): each
 // workgroup adds them up itself, workgroup 0 writes the counts, offsets and
-// tiles.  The passes of the one workgroup ran one after another, 7 us each:
+// tiles.  The passes of the one workgroup run one after another, 7 us each:
 // the launch took 58 us at 4096 tokens top-8 (8 passes) and 16 at 1021 (2), the
-// two take 10.8 + 11.6 and 4.9 + 8.7.
+// two took 10.8 + 11.6 and 4.9 + 8.7 with every activation row beside the counts.
+// A quarter of them there and the rest here (the counts take a third of the
+// placement's time): the call's 343.8 -> 340.4 us at 4096 tokens; 16384 tokens top-1
+// of 8 experts, H 128, whose rows take longer than the counts, 60.7 -> 53.6 (one
+// launch: 56.3).  A second pass of less than half is not worth the second launch
+// (top-8 of 8 experts, 5000 pairs 36.2 against 35.1, of 256 40.5 and 40.6; 8192 39.0
+// and 39.6, 48.3 and 50.8).
 template <bool SPLIT>
 __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
     const void* __restrict__ ids, int ids64, int64_t P, int32_t n_experts,
     int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ sorted_pairs,
     int32_t* __restrict__ pair_pos, int32_t* __restrict__ tiles, int32_t* __restrict__ n_tiles,
-    int32_t tile_tokens, int wide_tiles, const int32_t* __restrict__ hist, QuantRowsJob quant) {
+    int32_t tile_tokens, int wide_tiles, const int32_t* __restrict__ hist, int32_t n_pass,
+    int32_t quant_first, QuantRowsJob quant) {
   __shared__ int32_t cursor[kFastExperts];
   __shared__ uint16_t wcount[kFastWaves * kFastExperts];   // [wave][expert]
   __shared__ int32_t scratch[40];
   const int tid = threadIdx.x;
-  if (!SPLIT && blockIdx.x > 0) {
-    // the activation rows, four tokens per workgroup (a 256-thread quarter
-    // each, whole waves), beside workgroup 0's permutation; no barrier here
-    const int64_t t = 4 * static_cast<int64_t>(blockIdx.x - 1) + (tid >> 8);
+  const unsigned placing = SPLIT ? n_pass : 1;     // workgroups that place
+  if (blockIdx.x >= placing) {
+    // the activation rows from quant_first on, four tokens per workgroup (a
+    // 256-thread quarter each, whole waves), beside the permutation; no
+    // barrier here
+    const int64_t t = quant_first + 4 * static_cast<int64_t>(blockIdx.x - placing) + (tid >> 8);
     if (t < quant.tokens) quant_row(quant, t, tid & 255);
     return;
   }
@@ -302,7 +311,6 @@ __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
   __syncthreads();
   int32_t mine = 0, before = 0;    // expert tid's pairs, and those of earlier passes
   if constexpr (SPLIT) {
-    const int n_pass = static_cast<int>(gridDim.x);
     if (tid < E) {
 #pragma unroll 8
       for (int c = 0; c < n_pass; ++c) {
@@ -398,17 +406,17 @@ __global__ __launch_bounds__(kFastThreads) void permute_fast_kernel(
   }
 }
 
-// The expert counts of every placement pass, hist [n_pass][E], beside the
-// activation rows (four tokens per workgroup, as above).
+// The expert counts of every placement pass, hist [n_pass][E], beside the first
+// quant_end activation rows (four tokens per workgroup, as above).
 __global__ __launch_bounds__(kFastThreads) void permute_count_kernel(
     const void* __restrict__ ids, int ids64, int64_t P, int32_t n_experts, int32_t n_pass,
-    int32_t* __restrict__ hist, QuantRowsJob quant) {
+    int32_t* __restrict__ hist, int32_t quant_end, QuantRowsJob quant) {
   __shared__ int32_t cnt[kFastExperts];
   const int tid = threadIdx.x;
   const int c = static_cast<int>(blockIdx.x);
   if (c >= n_pass) {
     const int64_t t = 4 * static_cast<int64_t>(c - n_pass) + (tid >> 8);
-    if (t < quant.tokens) quant_row(quant, t, tid & 255);
+    if (t < quant_end) quant_row(quant, t, tid & 255);
     return;
   }
   int32_t v[kFastRounds];
@@ -554,22 +562,24 @@ int launch_permute(const void* ids, int ids64, int64_t P, int32_t n_experts, int
   static_assert(kFastThreads == 1024, "four 256-thread token slices per quantising workgroup");
   const QuantRowsJob q = quant ? *quant : QuantRowsJob{nullptr, 0, nullptr, nullptr, 0};
   const int64_t n_pass = (P + kFastPass - 1) / kFastPass;
-  if (n_experts <= kFastExperts && hist && n_pass > 1) {
-    hipLaunchKernelGGL(permute_count_kernel, dim3(static_cast<unsigned>(n_pass + (q.tokens + 3) / 4)),
+  if (n_experts <= kFastExperts && hist && P > kFastPass + kFastPass / 2) {
+    const int32_t early = (q.tokens / 4 + 3) & ~3;
+    const int32_t quant_end = early < q.tokens ? early : q.tokens;
+    hipLaunchKernelGGL(permute_count_kernel, dim3(static_cast<unsigned>(n_pass + (quant_end + 3) / 4)),
                        dim3(kFastThreads), 0, s, ids, ids64, P, n_experts,
-                       static_cast<int32_t>(n_pass), hist, q);
+                       static_cast<int32_t>(n_pass), hist, quant_end, q);
     const int rc = check_launch("moe_permute(count)");
     if (rc) return rc;
-    hipLaunchKernelGGL(permute_fast_kernel<true>, dim3(static_cast<unsigned>(n_pass)),
+    const int32_t late = q.tokens - quant_end;
+    hipLaunchKernelGGL(permute_fast_kernel<true>, dim3(static_cast<unsigned>(n_pass + (late + 3) / 4)),
                        dim3(kFastThreads), 0, s, ids, ids64, P, n_experts, counts, offsets,
                        sorted_pairs, pair_pos, tiles, n_tiles, tile_tokens, wide_tiles ? 1 : 0,
-                       hist, q);
+                       hist, static_cast<int32_t>(n_pass), quant_end, q);
   } else if (n_experts <= kFastExperts) {
     const unsigned grid = 1 + static_cast<unsigned>((q.tokens + 3) / 4);
     hipLaunchKernelGGL(permute_fast_kernel<false>, dim3(grid), dim3(kFastThreads), 0, s, ids, ids64, P,
                        n_experts, counts, offsets, sorted_pairs, pair_pos, tiles, n_tiles,
-                       tile_tokens, wide_tiles ? 1 : 0,
-                       nullptr, q);
+                       tile_tokens, wide_tiles ? 1 : 0, nullptr, 1, 0, q);
   } else {
     const unsigned grid = 1 + static_cast<unsigned>((q.tokens + 1) / 2);
     hipLaunchKernelGGL(wide_tiles ? permute_kernel<true> : permute_kernel<false>, dim3(grid),

@@ -201,6 +201,7 @@ def _device_experts(seed, E, H, I, dev):
     (40, 6, 4, 8192, 2048),      # the largest expert; weights read past the caches
     # several placement passes: the last of one pair, wide and streamed tiles, 1000 experts
     (4097, 2, 1, 256, 128), (1100, 300, 8, 128, 128), (1300, 1000, 7, 256, 128),
+    (6145, 3, 1, 256, 128), (8193, 2, 1, 256, 128),   # ... side by side, the last of one pair
     (4000, 1100, 8, 256, 128),   # wide tiles listed by the placement of more than 1024 experts
     # few rows per expert: 16-row tiles, most of one row; one expert with several
     (220, 450, 6, 256, 128), (40, 130, 8, 2048, 512), (64, 160, 6, 768, 384),
