@@ -76,7 +76,7 @@ inline bool glu_shape(int shape, int32_t inter) {
   return g >= 4 && inter % (32 * g) == 0;
 }
 
-// Calls on 16-row tiles: up to 5 rows per expert, of experts up to 2560 x 512.
+// Calls on 16-row tiles: up to 5 or 6 rows per expert, of experts up to 2560 x 512.
 // Half the LDS and a ring of 8 put four workgroups on a CU instead of two, with
 // as much in flight, so the last wave of items is shorter.  An expert picked by
 // more than 16 tokens has its weights read once per 16 rows, past the caches:
@@ -94,12 +94,14 @@ inline bool glu_shape(int shape, int32_t inter) {
 // the streamed one: at I 128, one K-block, too short for what it costs to start
 // (top-8 of 1000, even, 2 rows per expert: H 512 1.08, 1024 1.00, 2048 0.96, 4096
 // 0.91; uneven, 4 rows: 1.01, 0.96, 0.88, 0.79).
-constexpr int kSmallRowsPerExpert = 5;
+// Experts of a narrow hidden re-read little: up to 6 rows (512 x 512, top-8 of 256, 5.9
+// rows: even 1.09, uneven 1.05; 256 x 128, of 1500: 1.24 and 0.97; but 1024 x 256, of
+// 1000: 1.00 and 0.90).
 constexpr int32_t kSmallExpert = 2560 * 512;
 inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter) {
+  const int rows = hidden <= 512 ? 6 : 5;
   return hidden % 256 == 0 && hidden * inter <= kSmallExpert &&
-         (inter > 128 || hidden <= 1024) &&
-         P <= static_cast<int64_t>(kSmallRowsPerExpert) * n_experts;
+         (inter > 128 || hidden <= 1024) && P <= static_cast<int64_t>(rows) * n_experts;
 }
 
 // Calls on the wide tiles (grouped_wide.hip): by rows per expert, with w2 in

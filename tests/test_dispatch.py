@@ -122,10 +122,11 @@ def test_wide_plans_of_the_gpu_cases(rules, tiled):
 # do), and faster
 FEW_ROWS_NOT_SMALL = [(4096, 384, 256, 96), (3072, 512, 256, 80), (2048, 1024, 256, 80),
                       (8192, 512, 128, 80), (2048, 512, 256, 188), (2048, 512, 128, 92),
-                      (2048, 128, 1000, 500), (4096, 128, 1000, 250)]
+                      (2048, 128, 1000, 500), (4096, 128, 1000, 250), (1024, 256, 1000, 730)]
 FEW_ROWS_SMALL = [(2048, 512, 256, 29), (2048, 512, 256, 128), (2048, 512, 256, 160),
                   (1024, 1024, 256, 128), (2560, 512, 256, 58), (2560, 256, 256, 96),
-                  (512, 128, 1000, 250), (2048, 256, 256, 96)]
+                  (512, 128, 1000, 250), (2048, 256, 256, 96), (512, 512, 256, 188),
+                  (256, 128, 1500, 1024)]
 
 
 def test_sixteen_row_tiles(rules):
