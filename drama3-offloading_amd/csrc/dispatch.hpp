@@ -112,7 +112,10 @@ inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inte
 // Streamed over wide at 18 and 20 rows, mean (range) over 64 to 256 experts of
 // six shapes, evenly routed and by Zipf(1.1) popularity: tile order 0.99 (0.89
 // .. 1.19) and 1.01 (0.91 .. 1.18), row order 1.05 (0.88 .. 1.34) and 1.09 (0.88
-// .. 1.36).  Tile order, gate/up items of fewer than 16 K-blocks (their start
+// .. 1.36).  But 18 in tile order too of experts up to 256 MB:
+// over 73 calls of random sizes at 18 to 20 rows 1.09 (0.87 .. 1.41; 54 of them
+// above 1.03), against 1.01 of 256 to 512 MB and 1.00 above (even picks 0.93).
+// Tile order, gate/up items of fewer than 16 K-blocks (their start
 // and epilogue show) of experts well past the last-level cache, where the
 // streamed form runs at HBM's rate while most experts have one of its tiles:
 // H 1024, I 1024, 256 experts (805 MB), 20 rows 0.94 / 0.94, 28 0.98 / 0.99, 32 1.10 /
@@ -120,7 +123,7 @@ inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inte
 // 0.97, but of 256 experts (403 MB) 22 1.10 / 0.95; fewer than 8 K-blocks: H 256, I
 // 512, 1000 experts (393 MB), 22 0.78 / 0.83, 32 0.88 / 0.87, 64 1.26 / 1.21; H 768, I
 // 384, 512 (453 MB), 22 0.94 / 0.90, 32 1.02 / 0.92.
-constexpr int kWideRowsTiled = 20, kWideRowsRows = 18, kWideRowsShortItems = 32;
+constexpr int kWideRowsLow = 18, kWideRowsTiled = 20, kWideRowsShortItems = 32;
 constexpr int64_t kLastLevelCache = 256 << 20;   // bytes
 inline int64_t expert_set_bytes(int32_t n_experts, int32_t hidden, int32_t inter) {
   return 3LL * hidden * inter * n_experts;
@@ -130,7 +133,8 @@ inline bool enough_wide_rows(int64_t P, int32_t n_experts, int32_t hidden, int32
   const int64_t bytes = expert_set_bytes(n_experts, hidden, inter);
   const bool short_items = (hidden < 1024 && bytes > kLastLevelCache) ||
                            (hidden < 2048 && bytes > 2 * kLastLevelCache);
-  const int rows = !tiled ? kWideRowsRows : short_items ? kWideRowsShortItems : kWideRowsTiled;
+  const bool low = !tiled || bytes <= kLastLevelCache;
+  const int rows = low ? kWideRowsLow : short_items ? kWideRowsShortItems : kWideRowsTiled;
   return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(rows) * n_experts;
 }
 // ... and with enough of them to fill the chip: a call of a few tiles takes as

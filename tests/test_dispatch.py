@@ -85,13 +85,14 @@ def test_enough_items_take_the_wide_tiles(rules, case):
 # (hidden, inter, experts, rows of each, tile order): timed slower on the wide
 # tiles, evenly routed or by popularity, and faster
 FEW_ROWS_STREAMED = [
-    (2048, 512, 64, 18, True), (4096, 384, 192, 18, True), (1024, 512, 192, 18, True),
+    (2048, 512, 256, 18, True), (4096, 384, 192, 18, True), (1024, 512, 192, 18, True),
     (1024, 1024, 256, 18, True), (1024, 1024, 256, 24, True), (1024, 1024, 192, 24, True),
     (2048, 512, 256, 16, False), (1024, 1024, 256, 28, True), (1024, 512, 512, 24, True),
     (256, 512, 1000, 28, True), (768, 384, 512, 22, True), (512, 256, 1000, 24, True),
 ]
 ENOUGH_ROWS_WIDE = [
-    (2048, 512, 256, 20, True), (2048, 512, 64, 22, True), (2048, 1024, 64, 22, True),
+    (2048, 512, 256, 20, True), (2048, 512, 64, 18, True), (512, 512, 256, 18, True),
+    (2048, 512, 64, 22, True), (2048, 1024, 64, 22, True),
     (1024, 1024, 256, 32, True), (1024, 1024, 64, 24, True), (2048, 512, 256, 18, False),
     (1024, 512, 256, 22, True), (512, 512, 256, 22, True), (1024, 512, 1000, 22, False),
     (2560, 256, 64, 18, False), (1024, 1024, 256, 20, False), (2048, 512, 256, 31, False),
