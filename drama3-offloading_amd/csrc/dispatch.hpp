@@ -122,7 +122,10 @@ inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inte
 // 1.00, 40 1.27 / 1.05; H 1024, I 512, 512 experts (805 MB), 22 0.98 / 0.93, 32 1.07 /
 // 0.97, but of 256 experts (403 MB) 22 1.10 / 0.95; fewer than 8 K-blocks: H 256, I
 // 512, 1000 experts (393 MB), 22 0.78 / 0.83, 32 0.88 / 0.87, 64 1.26 / 1.21; H 768, I
-// 384, 512 (453 MB), 22 0.94 / 0.90, 32 1.02 / 0.92.
+// 384, 512 (453 MB), 22 0.94 / 0.90, 32 1.02 / 0.92.  One group of intermediate columns
+// (I 128) leaves the down items one K-block long: mean over random calls of 18 to 32
+// rows and 32 to 384 experts, H 2304 / 2560 / 3072 / 4096, tile order 1.13 / 1.04 / 1.01 /
+// 0.96, row order 1.15 / 1.01 / 0.95 / 0.88.
 constexpr int kWideRowsLow = 18, kWideRowsTiled = 20, kWideRowsShortItems = 32;
 constexpr int64_t kLastLevelCache = 256 << 20;   // bytes
 inline int64_t expert_set_bytes(int32_t n_experts, int32_t hidden, int32_t inter) {
@@ -131,10 +134,11 @@ inline int64_t expert_set_bytes(int32_t n_experts, int32_t hidden, int32_t inter
 inline bool enough_wide_rows(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter,
                              bool tiled) {
   const int64_t bytes = expert_set_bytes(n_experts, hidden, inter);
-  const bool short_items = (hidden < 1024 && bytes > kLastLevelCache) ||
-                           (hidden < 2048 && bytes > 2 * kLastLevelCache);
   const bool low = !tiled || bytes <= kLastLevelCache;
-  const int rows = low ? kWideRowsLow : short_items ? kWideRowsShortItems : kWideRowsTiled;
+  const bool short_items =
+      (inter == 128 && hidden >= (tiled ? 4096 : 3072)) ||
+      (!low && (hidden < 1024 || (hidden < 2048 && bytes > 2 * kLastLevelCache)));
+  const int rows = short_items ? kWideRowsShortItems : low ? kWideRowsLow : kWideRowsTiled;
   return hidden % kWideDownRows == 0 && P >= static_cast<int64_t>(rows) * n_experts;
 }
 // ... and with enough of them to fill the chip: a call of a few tiles takes as

@@ -89,6 +89,7 @@ FEW_ROWS_STREAMED = [
     (1024, 1024, 256, 18, True), (1024, 1024, 256, 24, True), (1024, 1024, 192, 24, True),
     (2048, 512, 256, 16, False), (1024, 1024, 256, 28, True), (1024, 512, 512, 24, True),
     (256, 512, 1000, 28, True), (768, 384, 512, 22, True), (512, 256, 1000, 24, True),
+    (3072, 128, 128, 24, False), (4096, 128, 256, 31, True),
 ]
 ENOUGH_ROWS_WIDE = [
     (2048, 512, 256, 20, True), (2048, 512, 64, 18, True), (512, 512, 256, 18, True),
@@ -96,6 +97,8 @@ ENOUGH_ROWS_WIDE = [
     (1024, 1024, 256, 32, True), (1024, 1024, 64, 24, True), (2048, 512, 256, 18, False),
     (1024, 512, 256, 22, True), (512, 512, 256, 22, True), (1024, 512, 1000, 22, False),
     (2560, 256, 64, 18, False), (1024, 1024, 256, 20, False), (2048, 512, 256, 31, False),
+    (4096, 128, 128, 32, False), (3072, 128, 256, 21, True),
+    (2304, 128, 128, 18, False),
 ]
 
 
