@@ -97,11 +97,18 @@ inline bool glu_shape(int shape, int32_t inter) {
 // Experts of a narrow hidden re-read little: up to 6 rows (512 x 512, top-8 of 256, 5.9
 // rows: even 1.09, uneven 1.05; 256 x 128, of 1500: 1.24 and 0.97; but 1024 x 256, of
 // 1000: 1.00 and 0.90).
+// In row order, whose loads use half lines, the re-reads cost more: there up to
+// kSmallRereadRows of rows per expert x hidden x inter.  Mean (lowest) over random
+// calls, even / Zipf(1.1) / those uneven picks, 2 to 2.5 Mi 1.08 (1.00) / 1.05 (0.91) / 1.00
+// (0.85), 2.5 to 3 1.08 (0.96) / 1.07 (1.00) / 0.96 (0.77), 3 to 4 1.04 (0.94) / 1.03 (0.90) /
+// 0.94 (0.79), above 1.06 (1.01) / 1.01 (0.95) / 0.95 (0.81).
 constexpr int32_t kSmallExpert = 2560 * 512;
-inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter) {
+constexpr int64_t kSmallRereadRows = 5 << 19;
+inline bool use_small(int64_t P, int32_t n_experts, int32_t hidden, int32_t inter, bool tiled) {
   const int rows = hidden <= 512 ? 6 : 5;
   return hidden % 256 == 0 && hidden * inter <= kSmallExpert &&
-         (inter > 128 || hidden <= 1024) && P <= static_cast<int64_t>(rows) * n_experts;
+         (inter > 128 || hidden <= 1024) && P <= static_cast<int64_t>(rows) * n_experts &&
+         (tiled || P * hidden * inter <= kSmallRereadRows * n_experts);
 }
 
 // Calls on the wide tiles (grouped_wide.hip): by rows per expert, with w2 in
@@ -215,7 +222,7 @@ inline GroupedPlan grouped_plan(int64_t P, int32_t n_experts, int32_t hidden, in
   }
   p.gate_up_shape = pick_shape(P, n_experts, 2 * inter, kGateUpShape);
   p.glu = glu_shape(p.gate_up_shape, inter);
-  p.tile_rows = p.glu && use_small(P, n_experts, hidden, inter) ? kSmallTileTok : kTileTok;
+  p.tile_rows = p.glu && use_small(P, n_experts, hidden, inter, tiled) ? kSmallTileTok : kTileTok;
   p.down_shape = pick_shape(P, n_experts, hidden, kDownShape);
   return p;
 }

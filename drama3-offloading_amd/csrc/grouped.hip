@@ -1,12 +1,13 @@
 // Grouped W8A8 expert FFN for many tokens (prefill, batched decode): token
 // rows are permuted into per-expert segments (permute.hip), the segments are
 // cut into tiles of up to 32 rows (16 or 64 in calls of few or many rows per
-// expert, grouped_plan in dispatch.hpp), every expert's weights are read from HBM once per tile, and the
-// results are un-permuted with the routing weights.
+// expert, grouped_plan in dispatch.hpp), every expert's weights are read from
+// HBM once per tile, and the results are un-permuted with the routing weights.
 //
 //   permute:     the token -> expert grouping and the tile list, and beside it
 //                x [T, H] bf16 -> xq [T, H] e4m3, xs [T, H/128] (per token;
-//                permute.hip): one launch, or two above 4096 pairs.
+//                permute.hip): one launch, or two above 6144 pairs of up to
+//                1024 experts.
 //   gate/up:     grouped_stream_kernel over (tile, rows of w13) work items,
 //                the tile's xq rows gathered by token.  In the GLU form (the
 //                default: items of whole 128-column groups) the epilogue

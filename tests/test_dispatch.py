@@ -140,6 +140,16 @@ def test_sixteen_row_tiles(rules):
     assert [rows[c] for c in FEW_ROWS_SMALL] == [16] * len(FEW_ROWS_SMALL)
 
 
+# the same in row order: uneven picks slower from 2.5 Mi of rows x hidden x inter
+@pytest.mark.parametrize("case, want", [((2048, 512, 256, 90), 32), ((1536, 512, 128, 74), 32),
+                                        ((2560, 512, 256, 91), 32), ((2048, 512, 256, 128), 32),
+                                        ((2048, 512, 256, 64), 16), ((2048, 256, 256, 96), 16),
+                                        ((1024, 512, 256, 128), 16)])
+def test_sixteen_row_tiles_in_row_order(rules, case, want):
+    H, I, E, T = case
+    assert grouped_plan(rules, T, E, 8, H, I, False).tile_rows == want
+
+
 def test_router_tiles(rules):
     """(experts, tokens) timed on MI355X, H 2048: slower with four tiles per
     workgroup (padded experts, CUs left idle at the end), and faster."""
