@@ -194,11 +194,13 @@ def _device_experts(seed, E, H, I, dev):
 
 
 @pytest.mark.parametrize("T,E,K,H,I", [
-    (18, 1, 1, 256, 128),        # the fewest rows of the wide tiles, one K-block of each projection
+    # too few items for the wide tiles: 32-row ones
+    (18, 1, 1, 256, 128),        # one K-block of down, two of gate/up
     (64, 1, 1, 2048, 512), (65, 1, 1, 512, 256), (129, 1, 1, 1024, 512),   # around whole tiles
     (100, 5, 3, 768, 384),       # a row block to spare, windows that end inside K
+    (40, 6, 4, 8192, 2048),      # the largest expert
+    # wide tiles
     (300, 16, 8, 2048, 512), (90, 4, 4, 4096, 1152),      # three windows of down
-    (40, 6, 4, 8192, 2048),      # the largest expert; weights read past the caches
     # several placement passes: the last of one pair, wide and streamed tiles, 1000 experts
     (4097, 2, 1, 256, 128), (1100, 300, 8, 128, 128), (1300, 1000, 7, 256, 128),
     (6145, 3, 1, 256, 128), (8193, 2, 1, 256, 128),   # ... side by side, the last of one pair
@@ -208,9 +210,9 @@ def _device_experts(seed, E, H, I, dev):
 ])
 @pytest.mark.parametrize("tiled", [False, True])
 def test_wide_tiles_equal_gemv(lib, dev, T, E, K, H, I, tiled):
-    """Many rows per expert or many pairs: token tiles of 64 rows, bit-identical to the
-    per-pair GEMV for full, ragged and single-row column tiles, an expert
-    without rows and picks of no expert (their tokens are NaN)."""
+    """Token tiles of 64, 32 and 16 rows, bit-identical to the per-pair GEMV for
+    full, ragged and single-row column tiles, an expert without rows and picks
+    of no expert (their tokens are NaN)."""
     from hostpool import RecordLayout
     import hipfetch
     devt = _device_experts(T + E, E, H, I, dev)
